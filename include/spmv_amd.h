@@ -183,6 +183,9 @@ int spmvx_matrix_arrays(spmvx_matrix A, const int32_t** rowptr_dev,
  * window number and an offset (2 instead of 4 bytes per entry); other blocks
  * keep the 32-bit indices.  A matrix's default is the 16-bit counterpart of
  * its dtype's default kernel when that covers at least half of the entries.
+ * Variants 8, 10 and 11 (those defaults) give every 64 rows to one wavefront
+ * where the rows are short and alike, and keep, for matrices whose rows use a
+ * short common list of column offsets, a mask per row in the indices' place.
  * The last variant, SPMVX_SLICED_VARIANT, is the sliced row-pattern layout:
  * for matrices whose rows repeat a few column-offset patterns (stencils), a
  * copy of the values is kept in 64-row slices with a 16-bit pattern id per

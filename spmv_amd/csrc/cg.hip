@@ -107,8 +107,8 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
            const X* b, X* x, int32_t kmax, Acc rtol, Acc* hist_dev, hipStream_t s)
 {
   Pattern& P = *A->pat;
-  const CsrView rb = csr_view(P, A->variant);
-  ensure_ws<X, Acc>(w, P, P.ncols, rb.nblocks);
+  const CsrView rb = csr_view(P, A->variant, sizeof(V));
+  ensure_ws<X, Acc>(w, P, P.ncols, rb.nparts);
   const int64_t n = P.nrows, ncols = P.ncols;
   auto* st = static_cast<CgState<Acc>*>(w.state);
   X* r = static_cast<X*>(w.r);
@@ -274,8 +274,11 @@ __global__ void add_correction(double* __restrict__ x, const float* __restrict__
 // ends.  In host code `scratch` names a host-side stand-in, not device
 // memory: its address on the current device comes from hipGetSymbolAddress,
 // looked up once per device and kept in scratch_addr.
+// The partial sums of csr_wave, whose number does not grow with the matrix,
+// have room of their own behind the SPMVX_CG_NOALLOC_SCRATCH_BYTES.
 constexpr size_t kNoAllocBytes = SPMVX_CG_NOALLOC_SCRATCH_BYTES;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
+constexpr size_t kNoAllocWave = sizeof(double) * kWaveMaxGrid;
+static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocWave];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mu;
@@ -336,7 +339,7 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
 {
   Pattern& P = *A->pat;
   const bool sliced = A->variant == kSlicedVariant;
-  const CsrView rbv = csr_view_built(P, A->variant);
+  const CsrView rbv = csr_view_built(P, A->variant, sizeof(double));
   const CsrView* rb = rbv.blocks ? &rbv : nullptr;
   SPMVX_REQUIRE(sliced || rb != nullptr,
                 "the row blocks of the matrix's kernel variant are not built");
@@ -357,7 +360,12 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   const int64_t hist_n = hist_host ? static_cast<int64_t>(kmax) + 1 : 0;
   const SlicedView sv = sliced ? sliced_view(A) : SlicedView{}; // built: no allocation
   const int64_t spw = (kSliceBS / kSlice) * (sliced ? sv.rpl : 1);
-  const int64_t nparts_max = sliced ? (sv.nslices + spw - 1) / spw : rb->nblocks;
+  // (csr_wave's count against the limit: one partial sum per 1024 rows or 8192
+  // entries, what csr_stream writes)
+  const bool wave = !sliced && rb->wave >= 0;
+  const int64_t nparts_max = sliced ? (sv.nslices + spw - 1) / spw
+                             : wave ? std::max((n + 1023) / 1024, (P.nnz + 8191) / 8192)
+                                    : rb->nparts;
   const NoAllocLayout L = noalloc_layout(n, ncols, nparts_max, g0, hist_n);
   if (L.total > kNoAllocBytes)
     throw Error(SPMVX_ERR_ARG, "spmvx_cg_noalloc: the solve needs " + std::to_string(L.total)
@@ -367,7 +375,7 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   double* r = reinterpret_cast<double*>(base + L.r);
   double* y = reinterpret_cast<double*>(base + L.y);
   double* p = reinterpret_cast<double*>(base + L.p);
-  double* part_s = reinterpret_cast<double*>(base + L.part_s);
+  double* part_s = reinterpret_cast<double*>(base + (wave ? kNoAllocBytes : L.part_s));
   double* part_0 = reinterpret_cast<double*>(base + L.part_0);
   double* part_1 = reinterpret_cast<double*>(base + L.part_1);
   auto* st = reinterpret_cast<CgState<double>*>(base + L.state);
@@ -519,10 +527,10 @@ int spmvx_ir_cg(spmvx_matrix A64, spmvx_matrix Alow, const double* b, double* x,
     SPMVX_REQUIRE((flags & ~SPMVX_IR_ADAPTIVE_INNER) == 0, "unknown refinement flags");
     hipStream_t s = as_stream(stream);
     const int64_t n = P.nrows;
-    const CsrView rb64 = csr_view(P, A64->variant);
-    ensure_ws<double, double>(A64->ws64, P, P.ncols, rb64.nblocks);
-    const CsrView rb32 = csr_view(P, Alow->variant);
-    ensure_ws<float, float>(Alow->ws32, P, P.ncols, rb32.nblocks);
+    const CsrView rb64 = csr_view(P, A64->variant, sizeof(double));
+    ensure_ws<double, double>(A64->ws64, P, P.ncols, rb64.nparts);
+    const CsrView rb32 = csr_view(P, Alow->variant, dtype_size(Alow->dtype));
+    ensure_ws<float, float>(Alow->ws32, P, P.ncols, rb32.nparts);
     CgWorkspace& w = A64->ws64;
     auto* st = static_cast<CgState<double>*>(w.state);
     double* r = static_cast<double*>(w.r);

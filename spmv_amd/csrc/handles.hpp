@@ -133,6 +133,17 @@ struct Pattern
   std::map<int, std::unique_ptr<SliceLayout>> slices; // by VW
   const RowPatterns* row_patterns();
   const SliceLayout& slice_layout(int vw);
+  // class of csr_wave that suits the rows (kWaveClasses), -1: none; found on
+  // first use
+  int wave_class();
+  int wave = -2;          // -2: not analysed yet
+  int ncu = 0;            // compute units of the device
+  int64_t widest_row = 0; // first row of the largest length
+  // row masks of csr_wave, built with the class's row blocks: a mask or length
+  // per row, (kind, first entry) per block, the list of column offsets
+  DevBuf wrows, wblocks, woffs;
+  bool masks_built = false, masked = false, all_masked = false;
+  void build_masks(const RowBlocks& rb);
   // the lazily built parts above are shared by every matrix made with
   // spmvx_matrix_create_like from one base, which callers may use from
   // different threads
@@ -148,14 +159,23 @@ std::vector<int2> row_blocks(const int32_t* rowptr, int64_t nrows, int64_t max_n
 // Default kernel variant of a value type (overridable with SPMVX_SPMV_VARIANT).
 int default_variant(int32_t dtype);
 
-// Row blocks used by the CSR kernel of variant `var`.
+// Stored entries and rows per row block of the CSR kernel of variant `var`:
+// csr_wave's where that kernel runs the variant.
+inline std::pair<int, int> variant_blocking(Pattern& P, int var)
+{
+  const int c = variant_wave(var) ? P.wave_class() : -1;
+  return c >= 0 ? std::pair<int, int>(wave_block_nnz(c), kWaveRows)
+                : std::pair<int, int>(variant_block_nnz(var), variant_block_rows(var));
+}
 inline const RowBlocks& variant_blocks(Pattern& P, int var)
 {
-  return P.blocks_for(variant_block_nnz(var), variant_block_rows(var));
+  const std::pair<int, int> k = variant_blocking(P, var);
+  return P.blocks_for(k.first, k.second);
 }
 inline const RowBlocks* built_variant_blocks(Pattern& P, int var)
 {
-  return P.find_blocks(variant_block_nnz(var), variant_block_rows(var));
+  const std::pair<int, int> k = variant_blocking(P, var);
+  return P.find_blocks(k.first, k.second);
 }
 
 // Builds the short column indices of a row blocking if missing (device
@@ -164,9 +184,10 @@ void build_short_index(Pattern& P, const RowBlocks& rb, int chunk);
 
 // The arrays a CSR kernel of variant `var` reads (blocks and, for the
 // short-index variants, the short indices are built if missing).
-CsrView csr_view(Pattern& P, int var);
+// vbytes: bytes of one stored value.
+CsrView csr_view(Pattern& P, int var, size_t vbytes);
 // The same without building anything: null blocks if they do not exist yet.
-CsrView csr_view_built(Pattern& P, int var);
+CsrView csr_view_built(Pattern& P, int var, size_t vbytes);
 
 // Builds the sliced layout of a matrix (row patterns, slices, values) if it
 // is missing; throws with the reason when the pattern is not eligible.

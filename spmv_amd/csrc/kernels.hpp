@@ -18,6 +18,7 @@
 // one XCD are adjacent and share x entries in that XCD's L2.
 #pragma once
 
+#include <algorithm>
 #include <initializer_list>
 
 #include <hip/hip_ext.h>
@@ -498,6 +499,8 @@ __global__ __launch_bounds__(BS) void csr_stream(
 // vec (consecutive entries per vector load), unroll (vector steps in flight),
 // non-temporal matrix loads, threads per workgroup (= rows per block at
 // most), short column indices}.  Variants 0-4 also take complex values.
+// Variants 8, 10 and 11, the 16-bit kernels that the matrices get by default,
+// run csr_wave instead where the matrix's rows suit it (wave_class).
 struct SpmvVariant
 {
   int chunk;
@@ -540,6 +543,7 @@ inline int variant_block_rows(int var)
     var = 0;
   return kVariants[var].bs;
 }
+inline bool variant_wave(int var) { return var == 8 || var == 10 || var == 11; }
 inline bool variant_short(int var) { return var >= 0 && var < kNumVariants && kVariants[var].i16; }
 
 // Device arrays of a CSR matrix for one row blocking: the CSR arrays, the
@@ -555,6 +559,16 @@ struct CsrView
   const int4* wbase;
   int32_t ncols;
   int short_kind; // 1: one base per block, 2: four windows per block
+  int wave;       // class of csr_wave (kWaveClasses) that runs the product, -1: csr_stream
+  int32_t burst;  // csr_wave: blocks per store of results, 0: each (WavePlan)
+  int32_t nrows;
+  int64_t nparts; // partial sums of a product with a reduction
+  // csr_wave: some block reads 16-bit indices; row masks (null: none), their
+  // blocks and column offsets
+  bool wcols = true;
+  const int32_t* wrows = nullptr;
+  const int2* wblocks = nullptr;
+  const int32_t* woffs = nullptr;
 };
 
 // Launches kernel with args on stream s; when ev0 / ev1 are given they
@@ -570,6 +584,13 @@ inline void launch_timed(void (*kernel)(KArgs...), dim3 grid, dim3 block, uint32
     kernel<<<grid, block, shmem, s>>>(static_cast<KArgs>(args)...);
 }
 
+} // namespace spmvx
+
+#include "wave.hpp"
+
+namespace spmvx
+{
+
 // Launches the SpMV kernel of variant `var` (blocks built with
 // variant_block_nnz/rows(var)); returns the number of partial sums written
 // (MODE != kPlain).  long_par: rows longer than a block are summed in
@@ -583,6 +604,12 @@ int64_t launch_csr_stream(int var, const CsrView& M, hipStream_t s, const V* val
 {
   if (M.nblocks <= 0)
     return 0;
+  if constexpr (!kIsComplex<V>)
+    if (M.wave >= 0)
+    {
+      launch_csr_wave<V, X, Acc, MODE>(M, s, val, x, y, b, partials, st, it, ev0, ev1);
+      return M.nparts;
+    }
   const dim3 grid(static_cast<unsigned>(M.nblocks));
 #define SPMVX_LAUNCH_IM(IMV)                                                                 \
   launch_timed(&csr_stream<V, X, Acc, MODE, C, VV, U, N, B, IMV>, grid, dim3(B), 0, s, ev0,   \

@@ -62,6 +62,52 @@ const RowBlocks* Pattern::find_blocks(int chunk, int rows)
   return it == blocks.end() ? nullptr : it->second.get();
 }
 
+// csr_wave gives every row of a group of 64 the same number of gathers (the
+// longest row's, in steps of KR): it suits rows that are short and alike.  The
+// first class whose blocks hold every group, if at most half as many gathers
+// again as stored entries are issued.
+int Pattern::wave_class()
+{
+  std::lock_guard<std::recursive_mutex> lock(lazy_mu);
+  if (wave != -2)
+    return wave;
+  wave = -1;
+  if (nnz == 0 || nrows > (int64_t(1) << 31) - (int64_t(1) << 16)) // 64-row steps past the end stay in 32 bits
+    return wave;
+  SPMVX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device));
+  int32_t widest = -1;
+  int64_t most = 0, slots[kNumWaveClasses] = {};
+  for (int64_t r = 0; r < nrows; r += kWaveRows)
+  {
+    const int64_t r1 = std::min<int64_t>(nrows, r + kWaveRows);
+    most = std::max<int64_t>(most, h_rowptr[r1] - h_rowptr[r]);
+    if (most > wave_block_nnz(kNumWaveClasses - 1))
+      return wave;
+    int32_t w = 0;
+    for (int64_t i = r; i < r1; ++i)
+    {
+      const int32_t len = h_rowptr[i + 1] - h_rowptr[i];
+      w = std::max(w, len);
+      if (len > widest || (len == widest && 2 * i <= nrows))
+      {
+        widest = len;
+        widest_row = i;
+      }
+    }
+    for (int c = 0; c < kNumWaveClasses; ++c)
+      slots[c] += static_cast<int64_t>((w + kWaveClasses[c].kr - 1) / kWaveClasses[c].kr)
+                  * kWaveClasses[c].kr * (r1 - r);
+  }
+  for (int c = 0; c < kNumWaveClasses; ++c)
+    if (most <= wave_block_nnz(c))
+    {
+      if (2 * slots[c] <= 3 * nnz)
+        wave = c;
+      break;
+    }
+  return wave;
+}
+
 const RowPatterns* Pattern::row_patterns()
 {
   std::lock_guard<std::recursive_mutex> lock(lazy_mu);
@@ -283,11 +329,90 @@ __global__ void short_encode(const int32_t* __restrict__ colidx, const int2* __r
       col16[k] = static_cast<uint16_t>((sel << 14) | off);
     }
     if (kind == 1 && threadIdx.x == 0)
-      wbase[bi] = make_int4(base, base, base, base);
+      // (read as four windows, they give the same columns)
+      wbase[bi] = make_int4(base, base + kWindow, base + 2 * kWindow, base + 3 * kWindow);
+  }
+}
+
+// Row masks of csr_wave, one wavefront per block of 64 rows: a row whose columns
+// are, in order, row + some of the n ascending offsets of the list has the mask
+// of those it uses.  Blocks whose rows all do: kind 1, masks; the others: kind
+// 0, lengths.  Counts the blocks without masks.
+__global__ void wave_masks(const int32_t* __restrict__ rowptr, const int32_t* __restrict__ colidx,
+                           int32_t nrows, const int32_t* __restrict__ offs, int32_t n,
+                           int32_t* __restrict__ rows, int2* __restrict__ blocks, int* count)
+{
+  const int32_t row = static_cast<int32_t>(blockIdx.x) * kWaveRows + static_cast<int32_t>(threadIdx.x);
+  const int32_t a = rowptr[row < nrows ? row : nrows], e = rowptr[row < nrows ? row + 1 : nrows];
+  uint32_t mask = 0;
+  int32_t k = a, q = 0;
+  while (k < e && q < n)
+  {
+    if (colidx[k] - row == offs[q])
+    {
+      mask |= 1u << q;
+      ++k;
+    }
+    ++q;
+  }
+  const bool all = __all(k == e);
+  rows[row] = all ? static_cast<int32_t>(mask) : e - a;
+  if (threadIdx.x == 0)
+  {
+    blocks[blockIdx.x] = make_int2(all ? 1 : 0, a);
+    if (!all)
+      atomicAdd(count, 1);
+    if (blockIdx.x + 1 == gridDim.x)
+      blocks[gridDim.x] = make_int2(0, rowptr[nrows]);
   }
 }
 
 } // namespace
+
+// The list of column offsets is the longest row's: for a stencil it holds every
+// row's.  (Of several, one near the middle: the first and last rows of periodic
+// operators wrap around.)  Kept when at least half of the blocks are masked (the others pay the
+// length sums on top of their indices).
+void Pattern::build_masks(const RowBlocks& rb)
+{
+  std::lock_guard<std::recursive_mutex> lock(lazy_mu);
+  if (masks_built)
+    return;
+  masks_built = true;
+  const int c = wave_class();
+  const int32_t a = h_rowptr[widest_row], n = h_rowptr[widest_row + 1] - a;
+  // gathers use 32-bit byte offsets into x, of up to 8 bytes per entry
+  if (c < 0 || n > kWaveClasses[c].kr || ncols > (int64_t(1) << 29) - 16
+      || nrows > (int64_t(1) << 29) - 16)
+    return;
+  std::vector<int32_t> offs(32, 0);
+  SPMVX_HIP(hipMemcpy(offs.data(), colidx.as<int32_t>() + a, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+  for (int32_t k = 0; k < n; ++k)
+    offs[k] -= static_cast<int32_t>(widest_row);
+  for (int32_t k = 1; k < n; ++k)
+    if (offs[k] <= offs[k - 1])
+      return;
+  DevBuf count;
+  count.ensure(sizeof(int));
+  woffs.ensure(sizeof(int32_t) * offs.size());
+  SPMVX_HIP(hipMemcpy(woffs.ptr, offs.data(), sizeof(int32_t) * offs.size(), hipMemcpyHostToDevice));
+  wrows.ensure(sizeof(int32_t) * static_cast<size_t>(rb.nblocks) * kWaveRows);
+  wblocks.ensure(sizeof(int2) * static_cast<size_t>(rb.nblocks + 1));
+  wave_masks<<<dim3(static_cast<unsigned>(rb.nblocks)), dim3(kWaveRows)>>>(
+      rowptr.as<int32_t>(), colidx.as<int32_t>(), static_cast<int32_t>(nrows), woffs.as<int32_t>(),
+      n, wrows.as<int32_t>(), wblocks.as<int2>(), count.as<int>());
+  check_launch("wave_masks");
+  int got = 0;
+  SPMVX_HIP(hipMemcpy(&got, count.ptr, sizeof(int), hipMemcpyDeviceToHost));
+  masked = 2 * static_cast<int64_t>(got) <= rb.nblocks;
+  all_masked = got == 0;
+  if (!masked)
+  {
+    wrows.release();
+    wblocks.release();
+    woffs.release();
+  }
+}
 
 void build_short_index(Pattern& P, const RowBlocks& rbc, int chunk)
 {
@@ -326,32 +451,58 @@ void build_short_index(Pattern& P, const RowBlocks& rbc, int chunk)
   rb.short_built = true;
 }
 
-CsrView csr_view(Pattern& P, int var)
+namespace
+{
+CsrView make_view(Pattern& P, const RowBlocks* rb, int var, size_t vbytes)
+{
+  CsrView M{P.rowptr.as<int32_t>(), P.colidx.as<int32_t>(), nullptr, 0, nullptr, nullptr,
+            static_cast<int32_t>(P.ncols), 0, -1, 0, static_cast<int32_t>(P.nrows), 0};
+  if (!rb)
+    return M;
+  M.blocks = rb->desc.as<int2>();
+  M.nblocks = M.nparts = rb->nblocks;
+  if (!variant_short(var))
+    return M;
+  M.col16 = rb->col16.as<uint16_t>();
+  M.wbase = rb->wbase.as<int4>();
+  M.short_kind = rb->short_kind;
+  M.wave = variant_wave(var) ? P.wave_class() : -1;
+  if (M.wave >= 0)
+  {
+    M.wcols = !P.masked || !P.all_masked;
+    const WavePlan plan = wave_plan(M.wave, static_cast<int>(vbytes), M.wcols, M.nblocks, P.ncu);
+    M.burst = plan.burst;
+    M.nparts = plan.grid;
+    if (P.masked)
+    {
+      M.wrows = P.wrows.as<int32_t>();
+      M.wblocks = P.wblocks.as<int2>();
+      M.woffs = P.woffs.as<int32_t>();
+    }
+  }
+  return M;
+}
+} // namespace
+
+CsrView csr_view(Pattern& P, int var, size_t vbytes)
 {
   const RowBlocks& rb = variant_blocks(P, var);
-  const bool sh = variant_short(var);
-  if (sh)
+  if (variant_short(var))
   {
-    build_short_index(P, rb, variant_block_nnz(var));
+    build_short_index(P, rb, variant_blocking(P, var).first);
     SPMVX_REQUIRE(rb.short_kind != 0 || P.nnz == 0,
                   "the matrix does not fit 16-bit column indices (a row block's columns "
                   "fall into more than four windows of 16384)");
+    if (variant_wave(var) && P.wave_class() >= 0)
+      P.build_masks(rb);
   }
-  return CsrView{P.rowptr.as<int32_t>(), P.colidx.as<int32_t>(), rb.desc.as<int2>(), rb.nblocks,
-                 sh ? rb.col16.as<uint16_t>() : nullptr, sh ? rb.wbase.as<int4>() : nullptr,
-                 static_cast<int32_t>(P.ncols), sh ? rb.short_kind : 0};
+  return make_view(P, &rb, var, vbytes);
 }
 
-CsrView csr_view_built(Pattern& P, int var)
+CsrView csr_view_built(Pattern& P, int var, size_t vbytes)
 {
   const RowBlocks* rb = built_variant_blocks(P, var);
-  const bool sh = variant_short(var);
-  if (!rb || (sh && !rb->short_built))
-    return CsrView{P.rowptr.as<int32_t>(), P.colidx.as<int32_t>(), nullptr, 0, nullptr, nullptr,
-                   static_cast<int32_t>(P.ncols), 0};
-  return CsrView{P.rowptr.as<int32_t>(), P.colidx.as<int32_t>(), rb->desc.as<int2>(), rb->nblocks,
-                 sh ? rb->col16.as<uint16_t>() : nullptr, sh ? rb->wbase.as<int4>() : nullptr,
-                 static_cast<int32_t>(P.ncols), sh ? rb->short_kind : 0};
+  return make_view(P, rb && variant_short(var) && !rb->short_built ? nullptr : rb, var, vbytes);
 }
 
 // Whether variant `var` of P can read 16-bit column indices (builds the
@@ -359,7 +510,9 @@ CsrView csr_view_built(Pattern& P, int var)
 bool fits_short(Pattern& P, int var)
 {
   const RowBlocks& rb = variant_blocks(P, var);
-  build_short_index(P, rb, variant_block_nnz(var));
+  build_short_index(P, rb, variant_blocking(P, var).first);
+  if (rb.short_kind != 0 && variant_wave(var) && P.wave_class() >= 0)
+    P.build_masks(rb);
   return rb.short_kind != 0;
 }
 
@@ -592,7 +745,7 @@ template <typename V, typename X, typename Acc>
 void launch_plain(int var, Pattern& P, const void* vals, const void* x, void* y, hipStream_t s,
                   int32_t long_par, hipEvent_t ev0, hipEvent_t ev1)
 {
-  const CsrView M = csr_view(P, var);
+  const CsrView M = csr_view(P, var, sizeof(V));
   launch_csr_stream<V, X, Acc, kPlain>(var, M, s, static_cast<const V*>(vals),
                                        static_cast<const X*>(x), static_cast<X*>(y), nullptr,
                                        nullptr, nullptr, 0, long_par, ev0, ev1);
@@ -925,7 +1078,7 @@ int spmvx_matrix_set_kernel(spmvx_matrix A, int32_t variant)
     if (v == kSlicedVariant)
       (void)sliced_view(A); // builds the layout or reports why it does not apply
     else
-      (void)csr_view(*A->pat, v); // row blocks (and short indices) built here
+      (void)csr_view(*A->pat, v, dtype_size(A->dtype)); // row blocks (and short indices) built here
     A->variant = v;
   });
 }
@@ -968,16 +1121,21 @@ int spmvx_matrix_get_kernel(spmvx_matrix A, int32_t* variant, char* name, int32_
       else
       {
         const SpmvVariant& k = kVariants[v];
-        d = std::string("csr_stream (") + std::to_string(k.bs) + " threads, chunk "
-            + std::to_string(k.chunk) + ", vec " + std::to_string(k.vec) + ", unroll "
-            + std::to_string(k.unroll) + (k.nt ? ", non-temporal" : "")
-            + (k.i16 ? std::string(", 16-bit column indices, ")
-                           + (built_variant_blocks(*A->pat, v)
-                                      && built_variant_blocks(*A->pat, v)->short_kind == 1
-                                  ? "one base per block"
-                                  : "four windows per block")
-                     : std::string())
-            + ")";
+        const int c = variant_wave(v) ? A->pat->wave_class() : -1;
+        if (c >= 0)
+          d = "csr_wave (one wavefront per 64 rows, " + std::to_string(kWaveClasses[c].kr)
+              + (A->pat->masked ? " column offsets and a mask per row, else " : " gathers at once, ");
+        else
+          d = std::string("csr_stream (") + std::to_string(k.bs) + " threads, chunk "
+              + std::to_string(k.chunk) + ", vec " + std::to_string(k.vec) + ", unroll "
+              + std::to_string(k.unroll) + (k.nt ? ", non-temporal" : "");
+        if (k.i16)
+        {
+          const RowBlocks* rb = built_variant_blocks(*A->pat, v);
+          d += std::string(c >= 0 ? "16-bit column indices, " : ", 16-bit column indices, ")
+               + (rb && rb->short_kind == 1 ? "one base per block" : "four windows per block");
+        }
+        d += ")";
       }
       const size_t n = std::min(d.size(), static_cast<size_t>(name_len - 1));
       std::memcpy(name, d.data(), n);
