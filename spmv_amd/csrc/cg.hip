@@ -7,6 +7,8 @@
 //   cg_update_r        r -= alpha y, partial ||r||^2             cg.cpp:66,69
 //   cg_beta_finalize   ||r||^2, beta, k, converged               cg.cpp:70-79
 //   cg_update_xp       x += alpha p, p = beta p + r              cg.cpp:65,76
+// Systems whose iterations are bound by launches run in one workgroup or in two
+// kernels per iteration instead (cg_small.hpp).
 // Every kernel returns immediately once the device-side `stopped` flag is
 // set, so the host replays a captured graph of a fixed number of iterations
 // and polls the flag between replays; the iteration count is exact.
@@ -16,6 +18,7 @@
 #include <mutex>
 #include <string>
 
+#include "cg_small.hpp"
 #include "handles.hpp"
 
 namespace spmvx
@@ -23,21 +26,39 @@ namespace spmvx
 namespace
 {
 
+// Whether an exchange of the column map leaves the direction as it is: no ghosts,
+// nothing to pack.
+bool without_exchange(const spmvx_l2gmap_s* m)
+{
+  return !m || (m->ghosts.empty() && m->indexbuf.empty());
+}
+
+// State of a solve on the device: the scalars, then the two slots of the
+// two-kernel iteration.
+template <typename Acc>
+struct CgDevice
+{
+  CgState<Acc> st;
+  CgSlot<Acc> slot[2];
+};
+
 template <typename X, typename Acc>
 void ensure_ws(CgWorkspace& w, const Pattern& P, int64_t ncols, int64_t nblocks)
 {
   const int64_t n = P.nrows;
-  if (w.mem.ptr && w.n == n && w.ncols == ncols && w.nblocks == nblocks && w.elem == sizeof(X))
+  const bool small = cg_is_small(P);
+  if (w.mem.ptr && w.n == n && w.ncols == ncols && w.nblocks == nblocks && w.elem == sizeof(X)
+      && (w.p2 != nullptr) == small)
     return;
   const int vgrid = vec_grid(n > ncols ? n : ncols);
   auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
   const size_t vec_n = al(sizeof(X) * static_cast<size_t>(n > 0 ? n : 1));
   const size_t vec_c = al(sizeof(X) * static_cast<size_t>(ncols > 0 ? ncols : 1));
-  const int64_t nb = nblocks > 0 ? nblocks : 1;
+  const int64_t nb = std::max<int64_t>({nblocks, small ? small_blocks(n) : 1, 1});
   const size_t red_s = al(sizeof(Acc) * static_cast<size_t>(nb));
   const size_t red_v = al(sizeof(Acc) * static_cast<size_t>(vgrid));
-  const size_t st_s = al(sizeof(CgState<Acc>));
-  const size_t total = 2 * vec_n + 3 * vec_c + red_s + 2 * red_v + st_s;
+  const size_t st_s = al(sizeof(CgDevice<Acc>));
+  const size_t total = 2 * vec_n + 4 * vec_c + (small ? vec_n : 0) + red_s + 2 * red_v + st_s;
   w.mem.release();
   char* base = static_cast<char*>(w.mem.ensure(total));
   size_t off = 0;
@@ -51,6 +72,8 @@ void ensure_ws(CgWorkspace& w, const Pattern& P, int64_t ncols, int64_t nblocks)
   w.p = take(vec_c);
   w.aux = take(vec_c);
   w.aux2 = take(vec_c);
+  w.x = take(vec_c);
+  w.p2 = small ? take(vec_n) : nullptr;
   w.red_spmv = take(red_s);
   w.red_vec0 = take(red_v);
   w.red_vec1 = take(red_v);
@@ -81,23 +104,23 @@ constexpr int kResidGrid = 1024;
 constexpr int kTailChunk = 4;   // iterations per graph near convergence
 
 // Whether the iterations still needed, extrapolated from the residual
-// decrease between two polls (k1, rho1) and the latest state, end within
+// decrease between two polls (k1, rho1) and the latest state (k, rho), end within
 // the replay in flight plus one more full chunk: then the next replays use
 // the short graph, so that fewer no-op iterations follow convergence.
-template <typename Acc>
-bool near_convergence(const CgState<Acc>& o, int32_t k1, double rho1, int32_t in_flight)
+bool near_convergence(int32_t k, double rho, double goal, int32_t k1, double rho1,
+                      int32_t in_flight)
 {
-  const double rho = static_cast<double>(o.rnorm_old);
-  if (k1 < 0 || o.k <= k1 || !(rho > 0.0) || !(rho < rho1))
+  if (k1 < 0 || k <= k1 || !(rho > 0.0) || !(rho < rho1))
     return false;
-  const double rate = std::log(rho / rho1) / static_cast<double>(o.k - k1); // < 0
-  const double need = std::log(static_cast<double>(o.rtol2) * static_cast<double>(o.rnorm0) / rho);
+  const double rate = std::log(rho / rho1) / static_cast<double>(k - k1); // < 0
+  const double need = std::log(goal / rho);
   return need / rate <= static_cast<double>(in_flight + kGraphChunk);
 }
 
 // Host driver of one CG solve.  x has ncols entries; b has nrows.
 // Chunks of kGraphChunk and kTailChunk iterations are captured once (per
-// matrix, x, history buffer and ghost map) and replayed; the kernels are
+// matrix, history buffer and ghost map; x is the workspace's, copied out at the
+// end, so that another x needs no new capture) and replayed; the kernels are
 // gated by the device state, so replays past convergence are no-ops.  Two
 // replays are kept in flight while the host polls the state of the older
 // one, switching to the short chunk when the residual decrease so far says
@@ -110,16 +133,31 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   const CsrView rb = csr_view(P, A->variant, sizeof(V));
   ensure_ws<X, Acc>(w, P, P.ncols, rb.nparts);
   const int64_t n = P.nrows, ncols = P.ncols;
-  auto* st = static_cast<CgState<Acc>*>(w.state);
+  auto* dev = static_cast<CgDevice<Acc>*>(w.state);
+  CgState<Acc>* st = &dev->st;
   X* r = static_cast<X*>(w.r);
   X* y = static_cast<X*>(w.y);
   X* p = static_cast<X*>(w.p);
+  X* xw = x == w.aux2 ? x : static_cast<X*>(w.x); // (the refinement's x is the workspace's)
   Acc* part_s = static_cast<Acc*>(w.red_spmv);
   Acc* part_0 = static_cast<Acc*>(w.red_vec0);
   Acc* part_1 = static_cast<Acc*>(w.red_vec1);
+  const V* csr_vals = static_cast<const V*>(A->values.ptr);
   const int vg = vec_grid(n);
   const int vgr = vg < kResidGrid ? vg : kResidGrid;
   const int g0 = vec_grid(ncols > n ? ncols : n);
+  auto* poll = static_cast<CgDevice<Acc>*>(w.poll.ensure(2 * sizeof(CgDevice<double>)));
+  const bool alone = without_exchange(col_map);
+  if (alone && cg_is_tiny(P))
+    for (bool first = true;; first = false)
+    {
+      launch_cg_tiny<V, X, Acc>(P, s, csr_vals, b, x, r, p, st, hist_dev, first, kmax, rtol * rtol);
+      SPMVX_HIP(hipMemcpyAsync(poll, dev, sizeof(CgDevice<Acc>), hipMemcpyDeviceToHost, s));
+      SPMVX_HIP(hipStreamSynchronize(s));
+      if (poll->st.stopped)
+        return poll->st.k;
+    }
+  const bool small = alone && cg_is_small(P);
   if (!w.stream)
   {
     SPMVX_HIP(hipStreamCreateWithFlags(&w.stream, hipStreamNonBlocking));
@@ -139,8 +177,20 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   const SlicedView sv = sliced ? sliced_view(A) : SlicedView{};
   const void* vals = sliced ? A->svalues.ptr : A->values.ptr;
 
-  // one CG iteration (cg.cpp:52-80); every kernel is gated by the state
-  auto iteration = [&](hipStream_t qq) {
+  // the caller's stream first (b and x may have just been written on it)
+  SPMVX_HIP(hipEventRecord(w.ev_in, s));
+  SPMVX_HIP(hipStreamWaitEvent(q, w.ev_in, 0));
+  cg_state_init<Acc><<<1, 1, 0, q>>>(st, kmax, rtol * rtol);
+  const SmallArgs<X, Acc> sm{r, y, {p, static_cast<X*>(w.p2)}, xw, part_s, part_1, st, dev->slot,
+                             hist_dev};
+  // one CG iteration (cg.cpp:52-80), the j-th of a graph; every kernel is
+  // gated by the state
+  auto iteration = [&](hipStream_t qq, int j) {
+    if (small)
+    {
+      launch_small_iteration<V, X, Acc>(P, qq, csr_vals, sm, j + 1);
+      return;
+    }
     if (col_map)
       l2gmap_update_async(col_map, vec_dtype, p, qq); // cg.cpp:55
     const int64_t nparts =
@@ -152,15 +202,16 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
     cg_alpha_finalize<Acc><<<1, kFinBS, 0, qq>>>(part_s, nparts, st, 1);
     cg_update_r<X, Acc><<<vgr, kVecBS, 0, qq>>>(n, r, y, part_1, st, 1);
     cg_beta_finalize<Acc><<<1, kFinBS, 0, qq>>>(part_1, vgr, st, hist_dev, 1);
-    cg_update_xp<X, Acc><<<vg, kVecBS, 0, qq>>>(n, x, p, r, st, 1);
+    cg_update_xp<X, Acc><<<vg, kVecBS, 0, qq>>>(n, xw, p, r, st, 1);
   };
 
   const void* halo = col_map ? col_map->d_halo.ptr : nullptr;
   const int32_t halo_dt = col_map ? col_map->halo_dtype : -2;
   const uint64_t map_id = col_map ? col_map->id : 0;
-  if (!w.exec || !w.exec_tail || w.g_x != x || w.g_hist != hist_dev || w.g_map != map_id
+  if (!w.exec || !w.exec_tail || w.g_x != xw || w.g_hist != hist_dev || w.g_map != map_id
       || w.g_halo != halo || w.g_halo_dtype != halo_dt || w.g_variant != A->variant
-      || w.g_long_rows != A->long_rows || w.g_mem != w.mem.ptr || w.g_values != vals)
+      || w.g_long_rows != A->long_rows || w.g_mem != w.mem.ptr || w.g_values != vals
+      || w.g_small != (small ? 1 : 0))
   {
     for (hipGraphExec_t* e : {&w.exec, &w.exec_tail})
     {
@@ -176,17 +227,17 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
     }
     w.graph = capture_graph(q, [&] {
       for (int j = 0; j < kGraphChunk; ++j)
-        iteration(q);
+        iteration(q, j);
     });
     check_launch("cg iteration capture");
     SPMVX_HIP(hipGraphInstantiate(&w.exec, w.graph, nullptr, nullptr, 0));
     w.graph_tail = capture_graph(q, [&] {
       for (int j = 0; j < kTailChunk; ++j)
-        iteration(q);
+        iteration(q, j);
     });
     check_launch("cg iteration capture");
     SPMVX_HIP(hipGraphInstantiate(&w.exec_tail, w.graph_tail, nullptr, nullptr, 0));
-    w.g_x = x;
+    w.g_x = xw;
     w.g_hist = hist_dev;
     w.g_map = map_id;
     w.g_halo = halo;
@@ -195,48 +246,55 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
     w.g_long_rows = A->long_rows;
     w.g_mem = w.mem.ptr;
     w.g_values = vals;
+    w.g_small = small ? 1 : 0;
   }
 
-  // the caller's stream first (b and x may have just been written on it)
-  SPMVX_HIP(hipEventRecord(w.ev_in, s));
-  SPMVX_HIP(hipStreamWaitEvent(q, w.ev_in, 0));
-  cg_state_init<Acc><<<1, 1, 0, q>>>(st, kmax, rtol * rtol);
-  cg_init<X, Acc><<<g0, kVecBS, 0, q>>>(n, ncols, b, x, r, p, part_0);
-  cg_init_finalize<Acc><<<1, kFinBS, 0, q>>>(part_0, g0, st, hist_dev);
+  if (small)
+    cg_small_init<X, Acc><<<small_partials(n), kSmallBS, 0, q>>>(n, b, xw, r, p, part_1, dev->slot);
+  else
+  {
+    cg_init<X, Acc><<<g0, kVecBS, 0, q>>>(n, ncols, b, xw, r, p, part_0);
+    cg_init_finalize<Acc><<<1, kFinBS, 0, q>>>(part_0, g0, st, hist_dev);
+  }
   check_launch("cg_init");
-  auto* poll = static_cast<CgState<Acc>*>(w.poll.ensure(2 * sizeof(CgState<double>)));
-  int32_t launched = 0;
+  // the two-kernel iteration completes iteration j in the first kernel of the
+  // next one: kmax + 1 of them
+  const int64_t need = static_cast<int64_t>(kmax) + (small ? 1 : 0);
+  int64_t launched = 0;
   int slot = 0, inflight = 0;
   int32_t chunk[2] = {0, 0};
-  bool stopped = kmax <= 0, tail = false;
+  bool stopped = need <= 0, tail = false;
   int32_t k1 = -1; // iteration and residual of the previous poll
   double rho1 = 0.0;
-  while (!stopped && launched < kmax)
+  while (!stopped && launched < need)
   {
     chunk[slot] = tail ? kTailChunk : kGraphChunk;
     SPMVX_HIP(hipGraphLaunch(tail ? w.exec_tail : w.exec, q));
     launched += chunk[slot];
-    SPMVX_HIP(hipMemcpyAsync(&poll[slot], st, sizeof(CgState<Acc>), hipMemcpyDeviceToHost, q));
+    SPMVX_HIP(hipMemcpyAsync(&poll[slot], dev, sizeof(CgDevice<Acc>), hipMemcpyDeviceToHost, q));
     SPMVX_HIP(hipEventRecord(w.ev_poll[slot], q));
     slot ^= 1;
     if (++inflight == 2)
     {
       SPMVX_HIP(hipEventSynchronize(w.ev_poll[slot])); // the older replay
-      const CgState<Acc> o = poll[slot];
-      stopped = o.stopped != 0;
+      const CgDevice<Acc> o = poll[slot];
+      const int32_t k = small ? o.slot[0].k : o.st.k;
+      const double rho = static_cast<double>(small ? o.slot[0].rr : o.st.rnorm_old);
+      stopped = (small ? o.slot[0].stopped : o.st.stopped) != 0;
       inflight = 1;
-      tail = near_convergence(o, k1, rho1, chunk[slot ^ 1]);
-      k1 = o.k;
-      rho1 = static_cast<double>(o.rnorm_old);
+      tail = near_convergence(k, rho,
+                              static_cast<double>(o.st.rtol2) * static_cast<double>(o.st.rnorm0),
+                              k1, rho1, chunk[slot ^ 1]);
+      k1 = k;
+      rho1 = rho;
     }
   }
-  CgState<Acc> fin{};
-  SPMVX_HIP(hipMemcpyAsync(A->host_flag.ensure(sizeof(CgState<Acc>)), st, sizeof(CgState<Acc>),
-                           hipMemcpyDeviceToHost, q));
+  if (xw != x)
+    SPMVX_HIP(hipMemcpyAsync(x, xw, sizeof(X) * static_cast<size_t>(ncols),
+                             hipMemcpyDeviceToDevice, q));
+  SPMVX_HIP(hipMemcpyAsync(poll, dev, sizeof(CgDevice<Acc>), hipMemcpyDeviceToHost, q));
   SPMVX_HIP(hipStreamSynchronize(q));
-  std::memcpy(&fin, A->host_flag.ptr, sizeof(fin));
-  (void)s;
-  return fin.k;
+  return small ? poll->slot[0].k : poll->st.k;
 }
 
 // ---------------------------------------------------------------- refinement
@@ -274,11 +332,15 @@ __global__ void add_correction(double* __restrict__ x, const float* __restrict__
 // ends.  In host code `scratch` names a host-side stand-in, not device
 // memory: its address on the current device comes from hipGetSymbolAddress,
 // looked up once per device and kept in scratch_addr.
-// The partial sums of csr_wave, whose number does not grow with the matrix,
-// have room of their own behind the SPMVX_CG_NOALLOC_SCRATCH_BYTES.
+// What run_cg's newer paths need beyond r, y, p and one partial sum per row
+// block has room of its own behind the SPMVX_CG_NOALLOC_SCRATCH_BYTES: the partial
+// sums of csr_wave (their number does not grow with the matrix) and of the
+// two-kernel iteration,
 constexpr size_t kNoAllocBytes = SPMVX_CG_NOALLOC_SCRATCH_BYTES;
 constexpr size_t kNoAllocWave = sizeof(double) * kWaveMaxGrid;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocWave];
+// the second direction of the two-kernel iteration
+constexpr size_t kNoAllocSmall = sizeof(double) * kSmallRows;
+static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocWave + kNoAllocSmall];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mu;
@@ -324,7 +386,7 @@ NoAllocLayout noalloc_layout(int64_t n, int64_t ncols, int64_t nparts, int vgrid
   L.part_s = take(8 * static_cast<size_t>(nparts > 0 ? nparts : 1));
   L.part_0 = take(8 * static_cast<size_t>(vgrid));
   L.part_1 = take(8 * static_cast<size_t>(vgrid));
-  L.state = take(sizeof(CgState<double>));
+  L.state = take(sizeof(CgDevice<double>));
   L.hist = take(8 * static_cast<size_t>(hist_n > 0 ? hist_n : 1));
   L.total = off;
   return L;
@@ -378,12 +440,28 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   double* part_s = reinterpret_cast<double*>(base + (wave ? kNoAllocBytes : L.part_s));
   double* part_0 = reinterpret_cast<double*>(base + L.part_0);
   double* part_1 = reinterpret_cast<double*>(base + L.part_1);
-  auto* st = reinterpret_cast<CgState<double>*>(base + L.state);
+  auto* dev = reinterpret_cast<CgDevice<double>*>(base + L.state);
+  CgState<double>* st = &dev->st;
   double* hist_dev = hist_host ? reinterpret_cast<double*>(base + L.hist) : nullptr;
   const void* vals = sliced ? A->svalues.ptr : A->values.ptr;
+  const double* csr_vals = static_cast<const double*>(A->values.ptr);
+  const bool alone = without_exchange(col_map);
+  const bool tiny = alone && cg_is_tiny(P);
+  const bool small = alone && !tiny && cg_is_small(P);
+  const SmallArgs<double, double> sm{
+      r,      y,
+      {p, reinterpret_cast<double*>(base + kNoAllocBytes + kNoAllocWave)},
+      x,      reinterpret_cast<double*>(base + kNoAllocBytes),
+      part_1, st,
+      dev->slot, hist_dev};
 
   // the iteration of run_cg (cg.cpp:52-80), every kernel gated by the state
-  auto iteration = [&]() {
+  auto iteration = [&](int j) {
+    if (small)
+    {
+      launch_small_iteration<double, double, double>(P, s, csr_vals, sm, j + 1);
+      return;
+    }
     if (col_map)
       l2gmap_update_async(col_map, SPMVX_F64, p, s); // cg.cpp:55
     const int64_t nparts =
@@ -398,31 +476,50 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
     cg_update_xp<double, double><<<vg, kVecBS, 0, s>>>(n, x, p, r, st, 1);
   };
 
-  cg_state_init<double><<<1, 1, 0, s>>>(st, kmax, rtol * rtol);
-  cg_init<double, double><<<g0, kVecBS, 0, s>>>(n, ncols, b, x, r, p, part_0);
-  cg_init_finalize<double><<<1, kFinBS, 0, s>>>(part_0, g0, st, hist_dev);
-  check_launch("cg_init");
-  int32_t launched = 0;
-  int32_t stopped = kmax <= 0 ? 1 : 0;
-  while (!stopped && launched < kmax)
+  if (!tiny)
+    cg_state_init<double><<<1, 1, 0, s>>>(st, kmax, rtol * rtol);
+  if (small)
+    cg_small_init<double, double><<<small_partials(n), kSmallBS, 0, s>>>(n, b, x, r, p, part_1,
+                                                                          dev->slot);
+  else if (!tiny)
   {
-    for (int j = 0; j < kGraphChunk; ++j)
-      iteration();
-    check_launch("cg iteration");
-    launched += kGraphChunk;
-    SPMVX_HIP(hipMemcpyAsync(&stopped, &st->stopped, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    cg_init<double, double><<<g0, kVecBS, 0, s>>>(n, ncols, b, x, r, p, part_0);
+    cg_init_finalize<double><<<1, kFinBS, 0, s>>>(part_0, g0, st, hist_dev);
+  }
+  check_launch("cg_init");
+  const int64_t need = static_cast<int64_t>(kmax) + (small || tiny ? 1 : 0);
+  int64_t launched = 0;
+  int32_t stopped = need <= 0 ? 1 : 0;
+  while (!stopped && launched < need)
+  {
+    if (tiny)
+    {
+      launch_cg_tiny<double, double, double>(P, s, csr_vals, b, x, r, p, st, hist_dev,
+                                             launched == 0, kmax, rtol * rtol);
+      launched += kTinySlice;
+    }
+    else
+    {
+      for (int j = 0; j < kGraphChunk; ++j)
+        iteration(j);
+      check_launch("cg iteration");
+      launched += kGraphChunk;
+    }
+    SPMVX_HIP(hipMemcpyAsync(&stopped, small ? &dev->slot[0].stopped : &st->stopped,
+                             sizeof(int32_t), hipMemcpyDeviceToHost, s));
     SPMVX_HIP(hipStreamSynchronize(s));
   }
-  CgState<double> fin{};
-  SPMVX_HIP(hipMemcpyAsync(&fin, st, sizeof(fin), hipMemcpyDeviceToHost, s));
+  CgDevice<double> fin{};
+  SPMVX_HIP(hipMemcpyAsync(&fin, dev, sizeof(fin), hipMemcpyDeviceToHost, s));
   SPMVX_HIP(hipStreamSynchronize(s));
+  const int32_t k = small ? fin.slot[0].k : fin.st.k;
   if (hist_host)
   {
-    SPMVX_HIP(hipMemcpyAsync(hist_host, hist_dev, sizeof(double) * (static_cast<size_t>(fin.k) + 1),
+    SPMVX_HIP(hipMemcpyAsync(hist_host, hist_dev, sizeof(double) * (static_cast<size_t>(k) + 1),
                              hipMemcpyDeviceToHost, s));
     SPMVX_HIP(hipStreamSynchronize(s));
   }
-  return fin.k;
+  return k;
 }
 
 // Argument checks shared by spmvx_cg and spmvx_cg_noalloc.
@@ -532,7 +629,7 @@ int spmvx_ir_cg(spmvx_matrix A64, spmvx_matrix Alow, const double* b, double* x,
     const CsrView rb32 = csr_view(P, Alow->variant, dtype_size(Alow->dtype));
     ensure_ws<float, float>(Alow->ws32, P, P.ncols, rb32.nparts);
     CgWorkspace& w = A64->ws64;
-    auto* st = static_cast<CgState<double>*>(w.state);
+    auto* st = &static_cast<CgDevice<double>*>(w.state)->st;
     double* r = static_cast<double*>(w.r);
     float* r32 = static_cast<float*>(Alow->ws32.aux);
     float* d32 = static_cast<float*>(Alow->ws32.aux2);

@@ -138,7 +138,8 @@ struct Pattern
   int wave_class();
   int wave = -2;          // -2: not analysed yet
   int ncu = 0;            // compute units of the device
-  int64_t widest_row = 0; // first row of the largest length
+  int64_t widest_row = 0; // a row of the largest length
+  int32_t longest = 0;    // entries of the longest row
   // row masks of csr_wave, built with the class's row blocks: a mask or length
   // per row, (kind, first entry) per block, the list of column offsets
   DevBuf wrows, wblocks, woffs;
@@ -289,6 +290,7 @@ struct CgWorkspace
   hipGraph_t graph_tail = nullptr; // kTailChunk iterations (near convergence)
   hipGraphExec_t exec_tail = nullptr;
   const void* g_x = nullptr;   // arguments the graphs were captured with
+  int32_t g_small = -1;
   const void* g_hist = nullptr;
   uint64_t g_map = 0; // id of the column map (0: none)
   const void* g_halo = nullptr;
@@ -306,6 +308,8 @@ struct CgWorkspace
   void* p = nullptr;
   void* aux = nullptr; // extra vector (refinement: residual / correction)
   void* aux2 = nullptr;
+  void* x = nullptr;  // the solution while iterating (the captured graphs' x)
+  void* p2 = nullptr; // second direction (two-kernel iterations)
   void* state = nullptr;
   void* red_spmv = nullptr;
   void* red_vec0 = nullptr;

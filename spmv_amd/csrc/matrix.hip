@@ -838,6 +838,8 @@ std::shared_ptr<Pattern> upload_pattern(int64_t nrows, int64_t ncols, int64_t nn
   if (nnz > 0)
     SPMVX_HIP(hipMemcpy(P->colidx.ptr, colidx, sizeof(int32_t) * nnz, hipMemcpyHostToDevice));
   P->h_rowptr.assign(rowptr, rowptr + nrows + 1);
+  for (int64_t i = 0; i < nrows; ++i)
+    P->longest = std::max(P->longest, rowptr[i + 1] - rowptr[i]);
   (void)variant_blocks(*P, default_variant(SPMVX_F64));
   return P;
 }
