@@ -4,9 +4,15 @@
 // spmv::cg (spmv/cg.cpp:50-80) in FP32 with NRHS right-hand sides at once.
 //
 // Design (gfx950):
-//   * one workgroup solves one whole system (all right-hand sides); all of
-//     its synchronisation is workgroup-local (__syncthreads), so workgroups
-//     never wait on each other and the grid always drains;
+//   * a team of workgroups solves one whole system (all right-hand sides), a slice
+//     of the rows each; a member is a queue slot, so that every member of a team
+//     that has started is running or next in its queue, waits are bounded and the
+//     grid always drains;
+//   * a team's sums travel as tagged words: a member stores {sequence, value} in one
+//     8-byte word per right-hand side and polls the others', one trip through
+//     memory instead of an arrival count and the sums behind it.  r, x and y are
+//     read by their own member only; p is read by all, so it alone is stored past
+//     the L2 of its XCD, and no fence has to write the L2 back at each exchange;
 //   * systems are pulled from a device work queue (atomic counter) in
 //     decreasing size order, so the largest start first (LPT schedule);
 //   * vectors are stored row-major [row][NRHS]: one 16-byte gather of p[c]
@@ -14,6 +20,11 @@
 //     iteration for all of them;
 //   * G lanes cooperate on a row (rows per wavefront = 64/G), chosen per
 //     system; G and the block size are picked by the autotuner.
+//
+// What bounds it (256 systems of 1000 to 50000 rows and 9.5 entries a row, 4 right-hand
+// sides, 66 ms; 131 ms with counted arrivals, fences and 16384 rows a member): latency of
+// the gathers of p with one workgroup per CU.  About 17 % of the time is their misses
+// (over gathers of the row's own p), 15 % the vector passes, 1.5 % the exchanges.
 #include <algorithm>
 #include <atomic>
 #include <cmath>
@@ -170,6 +181,31 @@ __device__ __forceinline__ VecD<NRHS> batch_resid(const int32_t* __restrict__ ro
   return tt;
 }
 
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v)
+{
+  const int o = __builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true);
+  return v + __int_as_float(o);
+}
+
+// Sum over the aligned group of G lanes, in all of them.  Lane i adds lane i ^ 1 and
+// i ^ 2 (quad permutations), then the mirrored lane of its 8 and of its 16, which
+// hold the other half's sum: register moves within the vector unit, where a shuffle
+// goes through the LDS pipe (G = 8 and 4 right-hand sides: 12 of them a row).
+template <int G>
+__device__ __forceinline__ float group_lanes_sum(float v)
+{
+  if constexpr (G >= 2)
+    v = dpp_add<0xB1>(v);
+  if constexpr (G >= 4)
+    v = dpp_add<0x4E>(v);
+  if constexpr (G >= 8)
+    v = dpp_add<0x141>(v);
+  if constexpr (G >= 16)
+    v = dpp_add<0x140>(v);
+  return v;
+}
+
 // y = A p over rows [r0, r1) with G lanes per row; returns this thread's
 // share of p.y (non-zero only in group leaders).  Each lane loads up to U
 // (colidx, value) pairs, then issues their U gathers of p, before
@@ -211,10 +247,8 @@ __device__ __forceinline__ VecN<NRHS> batch_spmv(const int32_t* __restrict__ row
           acc.v[j] += a[u] * pc[u].v[j];
     }
 #pragma unroll
-    for (int off = G / 2; off > 0; off >>= 1)
-#pragma unroll
-      for (int j = 0; j < NRHS; ++j)
-        acc.v[j] += __shfl_xor(acc.v[j], off, 64);
+    for (int j = 0; j < NRHS; ++j)
+      acc.v[j] = group_lanes_sum<G>(acc.v[j]);
     if (gl == 0)
     {
       stn<NRHS>(y + static_cast<int64_t>(row) * NRHS, acc);
@@ -231,6 +265,9 @@ __device__ __forceinline__ VecN<NRHS> batch_spmv(const int32_t* __restrict__ row
 // after about this many polls (a few seconds) instead of waiting forever; a
 // legitimate wait lasts at most one team member's solve of another system.
 constexpr unsigned kSpinLimit = 1u << 22;
+// Polls without a pause (an exchange in step takes a few); longer waits, a team
+// still gathering members, leave the memory alone in between.
+constexpr unsigned kSpinFast = 64;
 
 // Barrier among the W workgroups of one team (all of them are running: a
 // workgroup joins a team only by taking one of its slots from the queue).
@@ -263,32 +300,75 @@ __device__ __forceinline__ void team_barrier(unsigned* bar, unsigned target, int
   __syncthreads();
 }
 
-// Team-wide sum: member m stores its block sum in slot m of buffer `which`
-// (two buffers alternate), then every member adds the W slots in member
-// order (identical result in all members).
+// Team-wide sum of per-thread values: the workgroup's sum goes to the member's
+// words of buffer seq & 1, every member's are polled until they carry seq (all
+// words zeroed before the launch), summed in member order.  The two buffers
+// alternate: a member writes sequence seq + 2 only after every member has written
+// seq + 1, that is, has read seq.
 template <int NRHS>
-__device__ __forceinline__ VecN<NRHS> team_sum(VecN<NRHS> v, float* tred, int which, int W, int m,
-                                               unsigned* bar, unsigned& nbar, int* err,
-                                               float (*red)[16])
+__device__ __forceinline__ VecN<NRHS> team_total(VecN<NRHS> v, uint64_t* words, unsigned seq, int W,
+                                                 int m, int* err, float (*red)[16],
+                                                 float* total)
 {
   v = block_sum_n<NRHS>(v, red);
   if (W == 1)
     return v;
-  float* buf = tred + static_cast<int64_t>(which) * W * NRHS;
-  if (threadIdx.x == 0)
+  if (threadIdx.x < 64)
+  {
+    uint64_t* buf = words + static_cast<int64_t>(seq & 1u) * W * NRHS;
+    const int lane = threadIdx.x;
+    if (lane == 0)
+#pragma unroll
+      for (int j = 0; j < NRHS; ++j)
+        __hip_atomic_store(buf + m * NRHS + j,
+                           (static_cast<uint64_t>(seq) << 32) | __float_as_uint(v.v[j]),
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // lane q (q < W <= 64) polls member q's words
+    VecN<NRHS> o{};
+    unsigned spins = 0;
+    bool wait = lane < W;
+    while (__any(wait))
+    {
+      if (wait)
+      {
+        bool all = true;
+#pragma unroll
+        for (int j = 0; j < NRHS; ++j)
+        {
+          const uint64_t q = __hip_atomic_load(buf + lane * NRHS + j, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT);
+          all = all && static_cast<unsigned>(q >> 32) == seq;
+          o.v[j] = __uint_as_float(static_cast<uint32_t>(q));
+        }
+        if (all)
+          wait = false;
+        else if (++spins > kSpinLimit)
+        {
+          atomicExch(err, 1);
+          wait = false;
+        }
+        else if (spins > kSpinFast)
+          __builtin_amdgcn_s_sleep(8);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < NRHS; ++j)
-      buf[m * NRHS + j] = v.v[j];
-  team_barrier(bar, static_cast<unsigned>(W) * (++nbar), err);
-  VecN<NRHS> t{};
-  for (int q = 0; q < W; ++q)
+    {
+      const float t = wave_sum(lane < W ? o.v[j] : 0.0f);
+      if (lane == 0)
+        total[j] = t;
+    }
+  }
+  __syncthreads();
+  VecN<NRHS> t;
 #pragma unroll
-    for (int j = 0; j < NRHS; ++j)
-      t.v[j] += buf[q * NRHS + j];
+  for (int j = 0; j < NRHS; ++j)
+    t.v[j] = total[j];
   return t;
 }
 
-// team_sum in double (buffers of W * NRHS doubles, two alternating).
+// Team-wide sum in double: member m stores its block sum in slot m of buffer
+// `which` (two alternate), then every member adds the W slots in member order.
 template <int NRHS>
 __device__ __forceinline__ VecD<NRHS> team_sum_d(VecD<NRHS> v, double* tredd, int which, int W,
                                                  int m, unsigned* bar, unsigned& nbar, int* err,
@@ -309,6 +389,50 @@ __device__ __forceinline__ VecD<NRHS> team_sum_d(VecD<NRHS> v, double* tredd, in
     for (int j = 0; j < NRHS; ++j)
       t.v[j] += buf[q * NRHS + j];
   return t;
+}
+
+// Stores a row of p (or x) past this XCD's L2, so that members on other XCDs
+// read it after their own invalidation.
+template <int NRHS>
+__device__ __forceinline__ void stn_agent(float* p, const VecN<NRHS>& v)
+{
+  if constexpr (NRHS == 1)
+    __hip_atomic_store(p, v.v[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else
+#pragma unroll
+    for (int j = 0; j < NRHS; j += 2)
+    {
+      const uint64_t w = (static_cast<uint64_t>(__float_as_uint(v.v[j + 1])) << 32)
+                         | __float_as_uint(v.v[j]);
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(p + j), w, __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// Barrier of a team after stores past the L2 (stn_agent): they have completed
+// before the member's arrival (its waves wait for their stores at the first
+// workgroup barrier), and the caches are invalidated before any load behind it.
+__device__ __forceinline__ void team_publish(unsigned* bar, unsigned target, int* err)
+{
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0)
+  {
+    atomicAdd(bar, 1u);
+    unsigned spins = 0;
+    while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
+    {
+      if (++spins > kSpinLimit)
+      {
+        atomicExch(err, 1);
+        break;
+      }
+      if (spins > kSpinFast)
+        __builtin_amdgcn_s_sleep(8);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  __syncthreads();
 }
 
 // Index of the XCD (accelerator complex die) the calling wave runs on, from
@@ -333,9 +457,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
     const float* __restrict__ b, float* __restrict__ xu, float* __restrict__ xin,
     float* __restrict__ r, float* __restrict__ p, float* __restrict__ y, int32_t max_its,
     float rtol2, double rtol2d, int32_t* __restrict__ its_out, unsigned* queue, unsigned* bars,
-    float* tred_all, int* err)
+    double* tred_all, uint64_t* words_all, int* err)
 {
   __shared__ int2 job;
+  __shared__ float total[2][NRHS];
   __shared__ float red[NRHS][16];
   __shared__ double redd[NRHS][16];
   // queues are per XCD: members of one team share an L2; a workgroup whose
@@ -374,10 +499,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
     const int32_t hi = r0s + static_cast<int32_t>(ns * (m + 1) / W);
     const int g = gsel[s];
     unsigned* bar = bars + s;
-    float* tred = tred_all + tred_off[s];
-    // double sums after the float ones (an even float offset: 8-byte aligned)
-    double* tredd = reinterpret_cast<double*>(tred + 2 * static_cast<int64_t>(W) * NRHS);
-    unsigned nbar = 0;
+    // two alternating buffers of W x NRHS each
+    double* tredd = tred_all + tred_off[s];
+    uint64_t* words = words_all + tred_off[s];
+    unsigned nbar = 0, seq = 0;
     int nsum_d = 0;
 
     // x = 0, r = b, p = b, rr0 = ||b||^2 (cg.cpp:31-44); with a reordered
@@ -390,7 +515,7 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
       const VecN<NRHS> bi = ldn<NRHS>(b + static_cast<int64_t>(perm ? perm[i] : i) * NRHS);
       stn<NRHS>(x + o, VecN<NRHS>{});
       stn<NRHS>(r + o, bi);
-      stn<NRHS>(p + o, bi);
+      stn_agent<NRHS>(p + o, bi);
 #pragma unroll
       for (int j = 0; j < NRHS; ++j)
         rr.v[j] += bi.v[j] * bi.v[j];
@@ -400,7 +525,9 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
 #pragma unroll
     for (int j = 0; j < NRHS; ++j)
       bb.v[j] = static_cast<double>(rr.v[j]);
-    rr = team_sum<NRHS>(rr, tred, 0, W, m, bar, nbar, err, red); // also publishes p
+    if (W > 1)
+      team_publish(bar, static_cast<unsigned>(W) * (++nbar), err); // p complete
+    rr = team_total<NRHS>(rr, words, ++seq, W, m, err, red, total[seq & 1]);
     {
       VecD<NRHS> b2{};
       for (int32_t i = lo + static_cast<int32_t>(threadIdx.x); i < hi; i += blockDim.x)
@@ -443,7 +570,7 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
       case 8: pdy = batch_spmv<NRHS, 8>(rowptr, colidx, val, p, y, lo, hi); break;
       default: pdy = batch_spmv<NRHS, 16>(rowptr, colidx, val, p, y, lo, hi); break;
       }
-      pdy = team_sum<NRHS>(pdy, tred, 1, W, m, bar, nbar, err, red);
+      pdy = team_total<NRHS>(pdy, words, ++seq, W, m, err, red, total[seq & 1]);
       float alpha[NRHS];
 #pragma unroll
       for (int j = 0; j < NRHS; ++j)
@@ -465,7 +592,7 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
         }
         stn<NRHS>(r + o, ri);
       }
-      rn = team_sum<NRHS>(rn, tred, 0, W, m, bar, nbar, err, red);
+      rn = team_total<NRHS>(rn, words, ++seq, W, m, err, red, total[seq & 1]);
       float beta[NRHS];
       any = false;
 #pragma unroll
@@ -550,10 +677,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
           pi.v[j] = pi.v[j] * beta[j] + ri.v[j];
         }
         stn<NRHS>(x + o, xi);
-        stn<NRHS>(p + o, pi);
+        stn_agent<NRHS>(p + o, pi);
       }
       if (W > 1)
-        team_barrier(bar, static_cast<unsigned>(W) * (++nbar), err); // p complete
+        team_publish(bar, static_cast<unsigned>(W) * (++nbar), err); // p complete
     }
     if (perm)
     {
@@ -570,9 +697,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
   }
 }
 
-// queues = 0, every team's barrier counter = 0, err = 0 (a kernel, not a
+// queues = 0, every team's barrier counter and sum words = 0, err = 0 (a kernel, not a
 // memset node, so that graph replays are reliable)
-__global__ void batch_reset(unsigned* queue, int32_t nq, unsigned* bars, int32_t nsys, int* err)
+__global__ void batch_reset(unsigned* queue, int32_t nq, unsigned* bars, int32_t nsys, int* err,
+                            uint64_t* words, int64_t nwords)
 {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nq)
@@ -581,6 +709,8 @@ __global__ void batch_reset(unsigned* queue, int32_t nq, unsigned* bars, int32_t
     *err = 0;
   for (int32_t k = i; k < nsys; k += gridDim.x * blockDim.x)
     bars[k] = 0u;
+  for (int64_t k = i; k < nwords; k += gridDim.x * blockDim.x)
+    words[k] = 0u;
 }
 
 int pow2_ceil(int v)
@@ -606,14 +736,19 @@ struct spmvx_batch_s
   DevBuf perm;
   bool reordered = false;
   // team plan
-  DevBuf slots, qoff, team, tred_off, bars, tred, err;
+  DevBuf slots, qoff, team, tred_off, bars, tred, words, err;
+  int64_t nwords = 0;
   int32_t nslots = 0;
   int32_t nq = kNumXcd; // work queues, one per XCD
   bool plan_dirty = true;
   // launch configuration (autotuned)
   int32_t block = 1024;
   int32_t g_policy = 0;          // 0 = per system from the mean row length, else fixed G
-  int32_t rows_per_member = 16384; // team size = ceil(rows / rows_per_member), 0 = no teams
+  // Team size ceil(rows / rows_per_member), 0 = no teams; build_plan has the limits.
+  // 256 systems of 1000 to 50000 rows, 4 right-hand sides, to 1e-6: 16384 rows a member
+  // 126, 8192 81, 4096 66, 2048 66 ms (an exchange costs about 3 us, and the largest
+  // systems are the tail of the schedule).
+  int32_t rows_per_member = 4096;
   int grid = 0;
   // captured graph and the arguments it was captured with
   hipGraphExec_t exec = nullptr;
@@ -744,6 +879,23 @@ int batch_capacity(spmvx_batch_s* B)
   return std::max(1, per_cu) * std::max(1, ncu);
 }
 
+// Lanes per row from the mean row length: few enough that one pass over the rows
+// covers many of them (a pass is a chain of three loads: row bounds, entries, p),
+// enough that a row takes one or two batches of 4 entries per lane.  100 iterations
+// of 128 systems, 4 right-hand sides, G = 1 / 2 / 4 / 8 (ms): 5 entries a row
+// 11.4 / 12.0 / 14.5 / 19.9, 7: 12.6 / 12.6 / 15.1 / 20.9, 27: 65 / 40 / 27.7 / 31.9;
+// 256 systems of 9.5: 33.8 / 30.1 / 28.7 / 31.4; with G = 4 / 8 / 16, 49 entries:
+// 30.6 / 21.7 / 22.4, 81: 53 / 36.1 / 35.3.
+int lanes_for(int mean)
+{
+  if (mean < 10)
+    return pow2_ceil(std::max(1, mean / 4));
+  return mean <= 32 ? 4 : std::min(16, pow2_ceil(mean / 8));
+}
+
+constexpr int64_t kSmallTeam = 8, kWideMember = 16384;
+int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
 // Lanes per row (per system) and the team plan: systems in decreasing size
 // order (LPT), each split over W workgroups (W <= capacity / 2 so that a team
 // can always be completed by running workgroups), one queue slot per member.
@@ -766,12 +918,17 @@ void build_plan(spmvx_batch_s* B, int capacity)
       g[s] = static_cast<int8_t>(B->g_policy);
     else
     {
-      const int mean = rows > 0 ? static_cast<int>((nz + rows - 1) / rows) : 1;
-      g[s] = static_cast<int8_t>(std::min(16, pow2_ceil(std::max(1, mean / 4))));
+      g[s] = static_cast<int8_t>(
+          lanes_for(rows > 0 ? static_cast<int>((nz + rows - 1) / rows) : 1));
     }
     int64_t w = 1;
     if (B->rows_per_member > 0)
-      w = (rows + B->rows_per_member - 1) / B->rows_per_member;
+      // Members of less than kWideMember rows only in teams of up to kSmallTeam: a
+      // launch holds at most one gathering team per queue, 8 x 7 workgroups, so that
+      // launches on 4 streams (the hardware queues of a process) cannot fill the 256
+      // CUs with teams that all wait for members.
+      w = std::max(std::min(kSmallTeam, div_up(rows, B->rows_per_member)),
+                   div_up(rows, std::max<int64_t>(B->rows_per_member, kWideMember)));
     team[s] = static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>(w, wmax)));
   }
   // LPT: systems by decreasing work go to the XCD queue with the least work
@@ -798,7 +955,7 @@ void build_plan(spmvx_batch_s* B, int capacity)
   }
   std::vector<int64_t> off(nsys + 1, 0);
   for (int s = 0; s < nsys; ++s)
-    off[s + 1] = off[s] + 6LL * team[s] * B->nrhs; // 2 float + 2 double buffers
+    off[s + 1] = off[s] + 2LL * team[s] * B->nrhs;
   B->nslots = static_cast<int32_t>(slots.size());
   B->gsel.ensure(std::max(nsys, 1));
   B->team.ensure(4 * std::max(nsys, 1));
@@ -806,7 +963,9 @@ void build_plan(spmvx_batch_s* B, int capacity)
   B->slots.ensure(sizeof(int2) * std::max<size_t>(slots.size(), 1));
   B->qoff.ensure(4 * (nq + 1));
   SPMVX_HIP(hipMemcpy(B->qoff.ptr, qoff.data(), 4 * (nq + 1), hipMemcpyHostToDevice));
-  B->tred.ensure(4 * std::max<int64_t>(off[nsys], 1));
+  B->tred.ensure(8 * std::max<int64_t>(off[nsys], 1));
+  B->nwords = off[nsys];
+  B->words.ensure(8 * std::max<int64_t>(B->nwords, 1));
   B->bars.ensure(4 * std::max(nsys, 1));
   B->err.ensure(256);
   if (nsys)
@@ -829,7 +988,8 @@ void launch_batch(spmvx_batch_s* B, const float* b, float* x, int32_t max_its, d
   float* xin = y + vn; // x in the solver's row order (reordered batches)
   const int32_t* perm = B->reordered ? B->perm.as<int32_t>() : nullptr;
   batch_reset<<<std::max(1, std::min(64, (B->nsys + 255) / 256)), 256, 0, s>>>(
-      B->queue.as<unsigned>(), B->nq, B->bars.as<unsigned>(), B->nsys, B->err.as<int>());
+      B->queue.as<unsigned>(), B->nq, B->bars.as<unsigned>(), B->nsys, B->err.as<int>(),
+      B->words.as<uint64_t>(), B->nwords);
 #define SPMVX_BATCH(NR)                                                                        \
   batch_cg_kernel<NR><<<B->grid, B->block, 0, s>>>(                                           \
       B->rowptr.as<int32_t>(), B->colidx.as<int32_t>(), B->val.as<float>(),                    \
@@ -838,7 +998,7 @@ void launch_batch(spmvx_batch_s* B, const float* b, float* x, int32_t max_its, d
       B->tred_off.as<int64_t>(), B->gsel.as<int8_t>(), perm, b, x, xin, r, p, y, max_its,      \
       static_cast<float>(rtol * rtol), rtol * rtol,                                            \
       B->its.as<int32_t>(), B->queue.as<unsigned>(), B->bars.as<unsigned>(),                   \
-      B->tred.as<float>(), B->err.as<int>())
+      B->tred.as<double>(), B->words.as<uint64_t>(), B->err.as<int>())
   if (B->nrhs == 4)
     SPMVX_BATCH(4);
   else if (B->nrhs == 2)
