@@ -563,6 +563,7 @@ struct CsrView
   int32_t burst;  // csr_wave: blocks per store of results, 0: each (WavePlan)
   int32_t nrows;
   int64_t nparts; // partial sums of a product with a reduction
+  int64_t nnz = 0;
   // csr_wave: some block reads 16-bit indices; row masks (null: none), their
   // blocks and column offsets
   bool wcols = true;

@@ -460,6 +460,7 @@ CsrView make_view(Pattern& P, const RowBlocks* rb, int var, size_t vbytes)
   if (!rb)
     return M;
   M.blocks = rb->desc.as<int2>();
+  M.nnz = P.nnz;
   M.nblocks = M.nparts = rb->nblocks;
   if (!variant_short(var))
     return M;

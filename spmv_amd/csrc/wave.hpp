@@ -47,12 +47,15 @@ constexpr int kWaveRows = 64;
 // 1 KiB LDS loads (64 lanes of 16 bytes) that hold n entries of es bytes.
 __host__ __device__ constexpr int wave_loads(int n, int es) { return (n * es + 1023) / 1024; }
 
+// Cache bits of a buffer load: allocate as usual, or stream (non-temporal).
+constexpr int kLoadKeep = 0, kLoadStream = 2;
+
 // Requests `bytes` bytes (a multiple of 16, at most N KiB) from g (16-byte
 // aligned) into LDS; lanes past the end are out of the buffer's range and read
 // nothing.  The caller waits (lds_filled): the compiler does not order LDS
 // reads after these loads.
 typedef __attribute__((address_space(3))) char* lds_ptr;
-template <int N>
+template <int N, int AUX>
 __device__ __forceinline__ void lds_fill(const char* g, int32_t bytes, lds_ptr lds)
 {
   __amdgpu_buffer_rsrc_t r =
@@ -60,8 +63,7 @@ __device__ __forceinline__ void lds_fill(const char* g, int32_t bytes, lds_ptr l
   const int32_t off = static_cast<int32_t>(threadIdx.x) * 16;
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds + i * 1024, 16, off, i * 1024, 0,
-                                             2 /* non-temporal */);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds + i * 1024, 16, off, i * 1024, 0, AUX);
 }
 
 // Waits for every vector memory operation of this wavefront (the loads of
@@ -172,7 +174,7 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
               const int4* __restrict__ wbase, int32_t nrows, int32_t ncols,
               const V* __restrict__ val, const X* __restrict__ x, X* __restrict__ y,
               const X* __restrict__ b, Acc* __restrict__ partials, const CgState<Acc>* st,
-              int32_t it, WaveLds at, int32_t burst)
+              int32_t it, WaveLds at, int32_t burst, int32_t keep)
 {
   if (MODE != kPlain && !cg_live(st, it))
     return;
@@ -218,13 +220,18 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
       else if constexpr (MODE == kResid)
         xe = b[row < nrows ? row : nrows - 1];
     };
+    int32_t turn = 5 * j; // spreads the kept blocks over wavefronts and time
     auto fill = [&](int32_t a, int32_t e, int32_t masked) {
       const int32_t kb = a & ~(AL - 1);
       const int32_t n = (e - kb + AL - 1) & ~(AL - 1);
       if (!HM || !masked)
-        lds_fill<NX>(reinterpret_cast<const char*>(col16 + kb), n * 2, fill_at + at.col_at);
-      lds_fill<NV>(reinterpret_cast<const char*>(val + kb), n * static_cast<int32_t>(sizeof(V)),
-                   fill_at);
+        lds_fill<NX, kLoadStream>(reinterpret_cast<const char*>(col16 + kb), n * 2, fill_at + at.col_at);
+      const char* g = reinterpret_cast<const char*>(val + kb);
+      const int32_t bytes = n * static_cast<int32_t>(sizeof(V));
+      if ((turn++ & 31) < keep) // (wave_keep)
+        lds_fill<NV, kLoadKeep>(g, bytes, fill_at);
+      else
+        lds_fill<NV, kLoadStream>(g, bytes, fill_at);
     };
     int32_t of[KR]; // the list of column offsets, as byte offsets into x
 #pragma unroll
@@ -462,6 +469,28 @@ inline WavePlan wave_plan(int c, int vbytes, bool cols, int64_t nblocks, int ncu
   return WavePlan{0, std::min(nblocks, std::min(all, kWaveMaxGrid))};
 }
 
+// Of every 32 blocks, how many keep their values in the 256 MB last-level cache for
+// the next product of a solve; the others are streamed past it.  Loading all of a
+// larger matrix as usual would evict each line before its next use.  The kept share
+// is what fits beside the vectors in use (x, p, r and y of CG): from 160 to 240 MB in
+// all were within 2% of each other.  Below 64 MB the loads are left as streams
+// (27-point 64^3, 55 MB: kept 13.0, streamed 12.4 us).
+// Only CG's products do this: a product that may be the only one on its matrix loses
+// (27-point 160^3 after other work: 152 streamed, 156 us).
+// Streamed and by this rule, an iteration of FP64 CG, 27-point 112^3 (303 MB): 95 and
+// 83 us; FP32 CG, 7-point 256^3 (470 MB beside 268 MB of vectors): 3% less.  Repeated
+// products, us: 27-point 96^3 35.3 and 32.5, 128^3 78.4 and 72, 7-point 112^3 20.4 and
+// 19.0, FP32 256^3 121 and 115, BF16 93 and 88.
+constexpr double kKeepBytes = 208e6, kKeepLeast = 48e6, kKeepFrom = 64e6;
+inline int32_t wave_keep(int64_t nnz, size_t vbytes, double vector_bytes)
+{
+  const double bytes = static_cast<double>(nnz) * static_cast<double>(vbytes);
+  if (bytes < kKeepFrom)
+    return 0;
+  const double room = std::max(kKeepLeast, kKeepBytes - vector_bytes);
+  return std::min(32, static_cast<int32_t>(32.0 * room / bytes + 0.5));
+}
+
 // Launches csr_wave on M.nparts workgroups.
 template <typename V, typename X, typename Acc, int MODE>
 void launch_csr_wave(const CsrView& M, hipStream_t s, const V* val, const X* x, X* y, const X* b,
@@ -470,13 +499,16 @@ void launch_csr_wave(const CsrView& M, hipStream_t s, const V* val, const X* x, 
 {
   const dim3 grid(static_cast<unsigned>(M.nparts));
   const bool hm = M.wrows != nullptr;
+  const int32_t keep =
+      MODE == kDot ? wave_keep(M.nnz, sizeof(V), 4.0 * sizeof(X) * M.ncols) : 0;
   auto go = [&](auto im, auto masks, auto e, auto kr) {
     const WaveLds at = wave_lds(decltype(e)::value, sizeof(V), sizeof(X), M.wcols, M.burst);
     launch_timed(&csr_wave<V, X, Acc, MODE, decltype(im)::value, decltype(masks)::value,
                            decltype(e)::value, decltype(kr)::value>,
                  grid, dim3(kWaveRows), static_cast<uint32_t>(at.bytes), s, ev0, ev1,
                  hm ? M.wrows : M.rowptr, hm ? M.wblocks : M.blocks, M.woffs, M.col16, M.wbase,
-                 M.nrows, M.ncols, val, x, y, b, partials, st, it, at, M.burst);
+                 M.nrows, M.ncols, val, x, y, b, partials, st, it, at, M.burst,
+                 keep);
   };
   using std::integral_constant;
   auto kinds = [&](auto e, auto kr) {
