@@ -333,14 +333,16 @@ __global__ void add_correction(double* __restrict__ x, const float* __restrict__
 // memory: its address on the current device comes from hipGetSymbolAddress,
 // looked up once per device and kept in scratch_addr.
 // What run_cg's newer paths need beyond r, y, p and one partial sum per row
-// block has room of its own behind the SPMVX_CG_NOALLOC_SCRATCH_BYTES: the partial
-// sums of csr_wave (their number does not grow with the matrix) and of the
-// two-kernel iteration,
+// block of 1024 rows has room of its own behind the SPMVX_CG_NOALLOC_SCRATCH_BYTES:
+// the partial sums of csr_wave (their number does not grow with the matrix), of small
+// row blocks and of the two-kernel iteration,
 constexpr size_t kNoAllocBytes = SPMVX_CG_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kNoAllocWave = sizeof(double) * kWaveMaxGrid;
+constexpr size_t kNoAllocParts = 16384;
+static_assert(kNoAllocParts >= size_t(kWaveMaxGrid), "one partial sum per wavefront");
+constexpr size_t kNoAllocPart = sizeof(double) * kNoAllocParts;
 // the second direction of the two-kernel iteration
 constexpr size_t kNoAllocSmall = sizeof(double) * kSmallRows;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocWave + kNoAllocSmall];
+static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocPart + kNoAllocSmall];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mu;
@@ -422,12 +424,16 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   const int64_t hist_n = hist_host ? static_cast<int64_t>(kmax) + 1 : 0;
   const SlicedView sv = sliced ? sliced_view(A) : SlicedView{}; // built: no allocation
   const int64_t spw = (kSliceBS / kSlice) * (sliced ? sv.rpl : 1);
-  // (csr_wave's count against the limit: one partial sum per 1024 rows or 8192
-  // entries, what csr_stream writes)
-  const bool wave = !sliced && rb->wave >= 0;
+  // The partial sums of csr_wave and of the small row blocks that FP64 matrices get by
+  // default are behind the limit, where they fit, and against it counts what larger
+  // blocks write: one per 1024 rows or 8192 entries.
+  const bool behind = !sliced
+                      && (rb->wave >= 0
+                          || ((A->variant == 4 || A->variant == 9)
+                              && rb->nparts <= static_cast<int64_t>(kNoAllocParts)));
   const int64_t nparts_max = sliced ? (sv.nslices + spw - 1) / spw
-                             : wave ? std::max((n + 1023) / 1024, (P.nnz + 8191) / 8192)
-                                    : rb->nparts;
+                             : behind ? std::max((n + 1023) / 1024, (P.nnz + 8191) / 8192)
+                                      : rb->nparts;
   const NoAllocLayout L = noalloc_layout(n, ncols, nparts_max, g0, hist_n);
   if (L.total > kNoAllocBytes)
     throw Error(SPMVX_ERR_ARG, "spmvx_cg_noalloc: the solve needs " + std::to_string(L.total)
@@ -437,7 +443,7 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   double* r = reinterpret_cast<double*>(base + L.r);
   double* y = reinterpret_cast<double*>(base + L.y);
   double* p = reinterpret_cast<double*>(base + L.p);
-  double* part_s = reinterpret_cast<double*>(base + (wave ? kNoAllocBytes : L.part_s));
+  double* part_s = reinterpret_cast<double*>(base + (behind ? kNoAllocBytes : L.part_s));
   double* part_0 = reinterpret_cast<double*>(base + L.part_0);
   double* part_1 = reinterpret_cast<double*>(base + L.part_1);
   auto* dev = reinterpret_cast<CgDevice<double>*>(base + L.state);
@@ -450,7 +456,7 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   const bool small = alone && !tiny && cg_is_small(P);
   const SmallArgs<double, double> sm{
       r,      y,
-      {p, reinterpret_cast<double*>(base + kNoAllocBytes + kNoAllocWave)},
+      {p, reinterpret_cast<double*>(base + kNoAllocBytes + kNoAllocPart)},
       x,      reinterpret_cast<double*>(base + kNoAllocBytes),
       part_1, st,
       dev->slot, hist_dev};

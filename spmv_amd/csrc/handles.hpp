@@ -159,6 +159,8 @@ std::vector<int2> row_blocks(const int32_t* rowptr, int64_t nrows, int64_t max_n
 
 // Default kernel variant of a value type (overridable with SPMVX_SPMV_VARIANT).
 int default_variant(int32_t dtype);
+// The same for a pattern: small FP64 matrices get small row blocks.
+int plain_variant(const Pattern& P, int32_t dtype);
 
 // Stored entries and rows per row block of the CSR kernel of variant `var`:
 // csr_wave's where that kernel runs the variant.

@@ -532,33 +532,60 @@ int forced_variant()
 
 int default_variant(int32_t dtype)
 {
-  // measured best 32-bit-index CSR kernels on gfx950 for the stencil
-  // matrices: FP64 1024-thread workgroups staging 8192 entries (vec 2 x
-  // unroll 4), FP32 vec 4, BF16 vec 4 x unroll 2; SPMVX_SPMV_VARIANT overrides
+  // measured best 32-bit-index CSR kernels on gfx950 for large matrices: FP64
+  // 1024-thread workgroups staging 8192 entries (vec 2 x unroll 4), FP32 vec 4, BF16
+  // vec 4 x unroll 2; complex FP64 single entries, 4 in flight (16-byte values and
+  // gathers: 7-point 63^3 9.0 us against 10.1 with pairs, 160^3 129 against 145,
+  // 27-point 100^3 101 against 121), complex FP32 pairs (160^3 78.7 against 83.5);
+  // SPMVX_SPMV_VARIANT overrides
   const int forced = forced_variant();
-  if (dtype == SPMVX_C64 || dtype == SPMVX_C32) // variants 0-4 only (16 KB+ LDS products)
-    return forced >= 0 && forced <= 4 ? forced : 2;
+  if (is_complex(dtype)) // variants 0-4 only (16 KB+ LDS products)
+    return forced >= 0 && forced <= 4 ? forced : (dtype == SPMVX_C64 ? 1 : 2);
   if (forced >= 0)
     return forced;
   return dtype == SPMVX_F64 ? 5 : (dtype == SPMVX_F32 ? 3 : 4);
 }
 
+namespace
+{
+// FP64 matrices of at most this many entries get 2048-entry row blocks of 256
+// threads: blocks of 8192 entries are fewer than two per CU then, and a product is
+// the latency of its blocks.  Random power-law rows, 32-bit indices, kernel us with
+// 8192 and 2048 entries a block: 30 thousand entries 10.7 and 6.8, 287 thousand 14.8
+// and 8.0, 2.9 million 30 and 26 (repeated 24.8 and 20.6); 16-bit indices, 578
+// thousand 15.2 and 10.5, 4.2 million 30.7 and 31.0, 8 million 45.5 and 51.2.
+constexpr int64_t kSmallNnz = int64_t(1) << 22;
+bool small_blocks_suit(const Pattern& P, int32_t dtype)
+{
+  return dtype == SPMVX_F64 && P.nnz <= kSmallNnz && forced_variant() < 0;
+}
+} // namespace
+
+int plain_variant(const Pattern& P, int32_t dtype)
+{
+  return small_blocks_suit(P, dtype) ? 4 : default_variant(dtype);
+}
+
 int matrix_default_variant(spmvx_matrix_s* A)
 {
-  const int base = default_variant(A->dtype);
+  Pattern& P = *A->pat;
+  const int base = plain_variant(P, A->dtype);
   if (forced_variant() >= 0 || is_complex(A->dtype))
     return base;
   // the short-index kernel for the dtype when the matrix fits it (the
-  // analysis of the inspector, Matrix.cpp:43): FP64 the 16-bit counterpart
-  // of its default; FP32 and BF16 512-thread workgroups staging 4096 entries,
-  // FP32 with vec 4 x unroll 2 (variant 11), BF16 with 16-byte value loads
-  // (vec 8, variant 10): 1-5% (FP32) and 4-7% (BF16) faster per product on
-  // the 7- and 27-point stencils than 2048-entry blocks of 256 threads
-  const int sv = base == 5 ? 8 : (base == 3 ? 11 : (base == 4 ? 10 : -1));
-  Pattern& P = *A->pat;
-  if (sv < 0 || P.nnz == 0)
-    return base;
-  return fits_short(P, sv) ? sv : base;
+  // analysis of the inspector, Matrix.cpp:43); where the rows suit it, those
+  // whose products csr_wave runs.  Otherwise FP64 the 16-bit counterpart of
+  // its 32-bit one; FP32 and BF16 512-thread workgroups staging 4096 entries with
+  // 16-byte index loads (vec 8: FP32 bands of 20 million entries 65.5 us, vec 4 x
+  // unroll 2 74.8, 2048-entry blocks 85.4; BF16 57, 61 and 79)
+  const bool wave = P.wave_class() >= 0;
+  const int sv = A->dtype == SPMVX_F64 ? (!wave && small_blocks_suit(P, A->dtype) ? 9 : 8)
+                 : A->dtype == SPMVX_F32 && wave ? 11
+                                                 : 10;
+  if (P.nnz > 0 && fits_short(P, sv))
+    return sv;
+  (void)variant_blocks(P, base);
+  return base;
 }
 
 namespace
@@ -915,7 +942,7 @@ int transposed_variant(spmvx_matrix_s* A)
 {
   const int v = A->variant;
   if (v == kSlicedVariant || (variant_short(v) && !fits_short(*A->tpat, v)))
-    return default_variant(A->dtype);
+    return plain_variant(*A->tpat, A->dtype);
   return v;
 }
 

@@ -146,7 +146,7 @@ void build_transpose(spmvx_matrix_s* A, hipStream_t s)
                              sizeof(int32_t) * static_cast<size_t>(ncols + 1),
                              hipMemcpyDeviceToHost, s));
   SPMVX_HIP(hipStreamSynchronize(s));
-  (void)variant_blocks(*T, default_variant(A->dtype));
+  (void)variant_blocks(*T, plain_variant(*T, A->dtype));
   A->tpat = std::move(T);
 }
 
