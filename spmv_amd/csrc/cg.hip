@@ -1,12 +1,13 @@
 // Conjugate gradient on the device (spmv/cg.cpp:11-83) and the
 // mixed-precision iterative refinement built on it.
 //
-// One CG iteration = (ghost update) + 5 kernels, all scalars on the device:
-//   csr_stream<kDot> / sliced_spmv<kDot>  y = A p, partial p.y   cg.cpp:55-61
-//   cg_alpha_finalize  alpha = rnorm_old / p.y                   cg.cpp:62
-//   cg_update_r        r -= alpha y, partial ||r||^2             cg.cpp:66,69
-//   cg_beta_finalize   ||r||^2, beta, k, converged               cg.cpp:70-79
-//   cg_update_xp       x += alpha p, p = beta p + r              cg.cpp:65,76
+// One CG iteration = (ghost update) + 3 kernels, all scalars on the device:
+//   csr_wave / csr_stream / sliced_spmv<kDot>  y = A p, partial p.y  cg.cpp:55-61
+//   cg_fold_r   alpha = rnorm_old / p.y; r -= alpha y, partial ||r||^2  cg.cpp:62,66,69
+//   cg_fold_xp  ||r||^2, beta, k, converged; x += alpha p, p = beta p + r
+//                                                              cg.cpp:65,70-79
+// (with many partial sums of p.y, two kernels of one workgroup for the scalars and
+// cg_update_r, cg_update_xp).
 // Systems whose iterations are bound by launches run in one workgroup or in two
 // kernels per iteration instead (cg_small.hpp).
 // Every kernel returns immediately once the device-side `stopped` flag is
@@ -40,7 +41,84 @@ struct CgDevice
 {
   CgState<Acc> st;
   CgSlot<Acc> slot[2];
+  CgState<Acc> mid; // of an iteration between its two vector updates (cg_fold_r)
 };
+
+// ---------------------------------------------------------------- folded scalars
+// The vector updates with the sums before them: every workgroup adds the product's (or
+// the residual update's) partial sums for itself while its first vector loads are on
+// their way, and one workgroup writes the scalars for the next kernel.  A kernel never
+// writes the state it reads: cg_fold_r reads st and writes mid, cg_fold_xp reads mid
+// and writes st.
+// This takes the two one-workgroup kernels (4.6 us each, whatever the size) out of an
+// iteration and adds 1 to 2.4 us to the updates: FP64 us per iteration, 27-point 96^3
+// 54.1 to 49.1, 112^3 78.8 to 74.1, 180^3 337 to 333, 7-point 256^3 419 to 415; FP32
+// on BF16 values in the sliced layout, 7-point 160^3, 54.9 to 51.1.
+// All workgroups read all partial sums: taken up to kFoldBytes of them (8000 floats
+// in that last case; csr_wave leaves 1024 to 5120).
+constexpr int64_t kFoldBytes = 32768;
+
+template <typename X, typename Acc>
+__global__ __launch_bounds__(kVecBS) void cg_fold_r(int64_t n, X* __restrict__ r,
+                                                    const X* __restrict__ y,
+                                                    Acc* __restrict__ partials,
+                                                    const Acc* __restrict__ sums, int32_t nsums,
+                                                    const CgState<Acc>* st, CgState<Acc>* mid)
+{
+  const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+  if (st->stopped)
+  {
+    if (first)
+      mid->xp_pending = 0;
+    return;
+  }
+  __shared__ Acc red[16], redp[16];
+  Acc part = update_r<X, Acc>(n, r, y, [&] {
+    const Acc s = partials_sum<kVecBS, 16>(sums, nsums, redp);
+    const Acc alpha = st->rnorm_old / s;
+    if (first)
+    {
+      CgState<Acc> m = *st;
+      m.alpha = alpha;
+      m.xp_pending = 1;
+      *mid = m;
+    }
+    return static_cast<X>(alpha);
+  });
+  part = block_sum(part, red);
+  if (threadIdx.x == 0)
+    partials[blockIdx.x] = part;
+}
+
+template <typename X, typename Acc>
+__global__ __launch_bounds__(kVecBS) void cg_fold_xp(int64_t n, X* __restrict__ x,
+                                                     X* __restrict__ p, const X* __restrict__ r,
+                                                     const Acc* __restrict__ sums, int32_t nsums,
+                                                     CgState<Acc>* st, const CgState<Acc>* mid,
+                                                     Acc* __restrict__ hist)
+{
+  if (!mid->xp_pending)
+    return;
+  __shared__ Acc red[16];
+  update_xp<X>(n, x, p, r, [&](X& alpha, X& beta) {
+    const Acc s = partials_sum<kVecBS, 8>(sums, nsums, red);
+    const Acc b = s / mid->rnorm_old;
+    alpha = static_cast<X>(mid->alpha);
+    beta = static_cast<X>(b);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+    {
+      CgState<Acc> m = *mid;
+      m.beta = b;
+      m.rnorm_old = s;
+      ++m.k;
+      if (hist)
+        hist[m.k] = s;
+      m.converged = (s / m.rnorm0 < m.rtol2) ? 1 : 0;
+      m.stopped = (m.converged || m.k >= m.kmax) ? 1 : 0;
+      *st = m;
+    }
+  });
+}
 
 template <typename X, typename Acc>
 void ensure_ws(CgWorkspace& w, const Pattern& P, int64_t ncols, int64_t nblocks)
@@ -103,6 +181,27 @@ constexpr int kGraphChunk = 16; // iterations per captured graph
 constexpr int kResidGrid = 1024;
 constexpr int kTailChunk = 4;   // iterations per graph near convergence
 
+// The vector updates of an iteration behind its product (cg.cpp:59-79).
+template <typename X, typename Acc>
+void launch_updates(int64_t n, int64_t nparts, const Acc* part_s, Acc* part_1, X* x, X* p, X* r,
+                    const X* y, CgDevice<Acc>* dev, Acc* hist, hipStream_t s)
+{
+  const int vg = vec_grid(n);
+  const int vgr = vg < kResidGrid ? vg : kResidGrid;
+  CgState<Acc>* st = &dev->st;
+  if (nparts * static_cast<int64_t>(sizeof(Acc)) <= kFoldBytes)
+  {
+    cg_fold_r<X, Acc><<<vgr, kVecBS, 0, s>>>(n, r, y, part_1, part_s,
+                                             static_cast<int32_t>(nparts), st, &dev->mid);
+    cg_fold_xp<X, Acc><<<vg, kVecBS, 0, s>>>(n, x, p, r, part_1, vgr, st, &dev->mid, hist);
+    return;
+  }
+  cg_alpha_finalize<Acc><<<1, kFinBS, 0, s>>>(part_s, nparts, st, 1);
+  cg_update_r<X, Acc><<<vgr, kVecBS, 0, s>>>(n, r, y, part_1, st, 1);
+  cg_beta_finalize<Acc><<<1, kFinBS, 0, s>>>(part_1, vgr, st, hist, 1);
+  cg_update_xp<X, Acc><<<vg, kVecBS, 0, s>>>(n, x, p, r, st, 1);
+}
+
 // Whether the iterations still needed, extrapolated from the residual
 // decrease between two polls (k1, rho1) and the latest state (k, rho), end within
 // the replay in flight plus one more full chunk: then the next replays use
@@ -143,8 +242,6 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   Acc* part_0 = static_cast<Acc*>(w.red_vec0);
   Acc* part_1 = static_cast<Acc*>(w.red_vec1);
   const V* csr_vals = static_cast<const V*>(A->values.ptr);
-  const int vg = vec_grid(n);
-  const int vgr = vg < kResidGrid ? vg : kResidGrid;
   const int g0 = vec_grid(ncols > n ? ncols : n);
   auto* poll = static_cast<CgDevice<Acc>*>(w.poll.ensure(2 * sizeof(CgDevice<double>)));
   const bool alone = without_exchange(col_map);
@@ -199,10 +296,7 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
                : launch_csr_stream<V, X, Acc, kDot>(A->variant, rb, qq,
                                                     static_cast<const V*>(vals), p, y, nullptr,
                                                     part_s, st, 1, A->long_rows);
-    cg_alpha_finalize<Acc><<<1, kFinBS, 0, qq>>>(part_s, nparts, st, 1);
-    cg_update_r<X, Acc><<<vgr, kVecBS, 0, qq>>>(n, r, y, part_1, st, 1);
-    cg_beta_finalize<Acc><<<1, kFinBS, 0, qq>>>(part_1, vgr, st, hist_dev, 1);
-    cg_update_xp<X, Acc><<<vg, kVecBS, 0, qq>>>(n, xw, p, r, st, 1);
+    launch_updates<X, Acc>(n, nparts, part_s, part_1, xw, p, r, y, dev, hist_dev, qq);
   };
 
   const void* halo = col_map ? col_map->d_halo.ptr : nullptr;
@@ -418,8 +512,6 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
                   "halo dtype differs from the vector dtype");
   }
   const int64_t n = P.nrows, ncols = P.ncols;
-  const int vg = vec_grid(n);
-  const int vgr = vg < kResidGrid ? vg : kResidGrid;
   const int g0 = vec_grid(ncols > n ? ncols : n);
   const int64_t hist_n = hist_host ? static_cast<int64_t>(kmax) + 1 : 0;
   const SlicedView sv = sliced ? sliced_view(A) : SlicedView{}; // built: no allocation
@@ -476,10 +568,7 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
                : launch_csr_stream<double, double, double, kDot>(
                      A->variant, *rb, s, static_cast<const double*>(vals), p, y, nullptr, part_s,
                      st, 1, A->long_rows);
-    cg_alpha_finalize<double><<<1, kFinBS, 0, s>>>(part_s, nparts, st, 1);
-    cg_update_r<double, double><<<vgr, kVecBS, 0, s>>>(n, r, y, part_1, st, 1);
-    cg_beta_finalize<double><<<1, kFinBS, 0, s>>>(part_1, vgr, st, hist_dev, 1);
-    cg_update_xp<double, double><<<vg, kVecBS, 0, s>>>(n, x, p, r, st, 1);
+    launch_updates<double, double>(n, nparts, part_s, part_1, x, p, r, y, dev, hist_dev, s);
   };
 
   if (!tiny)

@@ -73,20 +73,22 @@ __device__ __forceinline__ T group_total(T v, T* red)
 
 // Sum of n partials by every workgroup for itself (blockDim.x = BS): each
 // thread's loads all in flight, fixed order, valid in all threads.
-template <int BS, typename Acc>
+template <int BS, int U = 4, typename Acc>
 __device__ __forceinline__ Acc partials_sum(const Acc* __restrict__ part, int32_t n, Acc* red)
 {
   Acc s0 = Acc(0), s1 = Acc(0);
-  for (int32_t i = threadIdx.x; i < n; i += 4 * BS)
+  for (int32_t i = threadIdx.x; i < n; i += U * BS)
   {
-    Acc v[4];
+    Acc v[U];
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+    for (int u = 0; u < U; ++u)
       v[u] = i + u * BS < n ? part[i + u * BS] : Acc(0);
-    s0 += v[0];
-    s1 += v[1];
-    s0 += v[2];
-    s1 += v[3];
+#pragma unroll
+    for (int u = 0; u < U; u += 2)
+    {
+      s0 += v[u];
+      s1 += v[u + 1];
+    }
   }
   return group_total<BS / 64>(s0 + s1, red);
 }

@@ -1081,6 +1081,60 @@ __global__ __launch_bounds__(kFinBS) void sum_finalize(const Acc* __restrict__ p
     st->last = s;
 }
 
+// r -= alpha y (cg.cpp:66); this thread's share of ||r||^2.  coefficient() gives alpha,
+// called once, with the thread's first loads on their way.
+template <typename X, typename Acc, typename F>
+__device__ __forceinline__ Acc update_r(int64_t n, X* __restrict__ r, const X* __restrict__ y,
+                                        F&& coefficient)
+{
+  Acc part = Acc(0);
+  constexpr int N = Pack16<X>::N;
+  const int64_t gid = blockIdx.x * static_cast<int64_t>(kVecBS) + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kVecBS;
+  const bool packed = aligned16(r, y);
+  const int64_t npk = packed ? n / N : 0; // 16-byte packs
+  // two packs per thread and step, both loaded before either is used (the
+  // second re-reads the first when past the end; stored only when in range)
+  Pack16<X> ra{}, ya{}, rb{}, yb{};
+  auto load = [&](int64_t q) {
+    const int64_t q2 = q + stride < npk ? q + stride : q;
+    ra = ld16(r + q * N), ya = ld16<kStreamLastRead<X>>(y + q * N);
+    rb = ld16(r + q2 * N), yb = ld16<kStreamLastRead<X>>(y + q2 * N);
+  };
+  if (gid < npk)
+    load(gid);
+  const X alpha = coefficient();
+  for (int64_t q = gid; q < npk; q += 2 * stride)
+  {
+    if (q != gid)
+      load(q);
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+    {
+      ra.v[e] = ra.v[e] - alpha * ya.v[e];
+      part += static_cast<Acc>(ra.v[e]) * static_cast<Acc>(ra.v[e]);
+    }
+    st16(r + q * N, ra);
+    if (q + stride < npk)
+    {
+#pragma unroll
+      for (int e = 0; e < N; ++e)
+      {
+        rb.v[e] = rb.v[e] - alpha * yb.v[e];
+        part += static_cast<Acc>(rb.v[e]) * static_cast<Acc>(rb.v[e]);
+      }
+      st16(r + (q + stride) * N, rb);
+    }
+  }
+  for (int64_t i = npk * N + gid; i < n; i += stride)
+  {
+    const X ri = r[i] - alpha * ld_stream<kStreamLastRead<X>>(y + i);
+    r[i] = ri;
+    part += static_cast<Acc>(ri) * static_cast<Acc>(ri);
+  }
+  return part;
+}
+
 // r -= alpha y; partial ||r||^2 (cg.cpp:66,69)
 template <typename X, typename Acc>
 __global__ __launch_bounds__(kVecBS) void cg_update_r(int64_t n, X* __restrict__ r,
@@ -1091,50 +1145,7 @@ __global__ __launch_bounds__(kVecBS) void cg_update_r(int64_t n, X* __restrict__
   if (!cg_live(st, it))
     return;
   __shared__ Acc red[16];
-  const X alpha = static_cast<X>(st->alpha);
-  Acc part = Acc(0);
-  constexpr int N = Pack16<X>::N;
-  const int64_t gid = blockIdx.x * static_cast<int64_t>(kVecBS) + threadIdx.x;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kVecBS;
-  int64_t done = 0; // elements covered by the 16-byte passes
-  if (aligned16(r, y))
-  {
-    // two 16-byte packs per thread and step, both loaded before either is
-    // used (the second re-reads the first when past the end; stored only
-    // when in range)
-    const int64_t npk = n / N;
-    for (int64_t q = gid; q < npk; q += 2 * stride)
-    {
-      const bool two = q + stride < npk;
-      const int64_t q2 = two ? q + stride : q;
-      Pack16<X> ra = ld16(r + q * N), ya = ld16<kStreamLastRead<X>>(y + q * N);
-      Pack16<X> rb = ld16(r + q2 * N), yb = ld16<kStreamLastRead<X>>(y + q2 * N);
-#pragma unroll
-      for (int e = 0; e < N; ++e)
-      {
-        ra.v[e] = ra.v[e] - alpha * ya.v[e];
-        part += static_cast<Acc>(ra.v[e]) * static_cast<Acc>(ra.v[e]);
-      }
-      st16(r + q * N, ra);
-      if (two)
-      {
-#pragma unroll
-        for (int e = 0; e < N; ++e)
-        {
-          rb.v[e] = rb.v[e] - alpha * yb.v[e];
-          part += static_cast<Acc>(rb.v[e]) * static_cast<Acc>(rb.v[e]);
-        }
-        st16(r + q2 * N, rb);
-      }
-    }
-    done = npk * N;
-  }
-  for (int64_t i = done + gid; i < n; i += stride)
-  {
-    const X ri = r[i] - alpha * ld_stream<kStreamLastRead<X>>(y + i);
-    r[i] = ri;
-    part += static_cast<Acc>(ri) * static_cast<Acc>(ri);
-  }
+  Acc part = update_r<X, Acc>(n, r, y, [&] { return static_cast<X>(st->alpha); });
   part = block_sum(part, red);
   if (threadIdx.x == 0)
     partials[blockIdx.x] = part;
@@ -1164,8 +1175,50 @@ __global__ __launch_bounds__(kFinBS) void cg_beta_finalize(const Acc* __restrict
   }
 }
 
-// x += alpha p; p = beta p + r (cg.cpp:65,76): runs iff this iteration
-// completed its residual update (also on the iteration that stops).
+// x += alpha p; p = beta p + r (cg.cpp:65,76).  coefficients(alpha, beta) sets both,
+// called once, with the thread's first loads on their way.
+template <typename X, typename F>
+__device__ __forceinline__ void update_xp(int64_t n, X* __restrict__ x, X* __restrict__ p,
+                                          const X* __restrict__ r, F&& coefficients)
+{
+  constexpr int N = Pack16<X>::N;
+  const int64_t gid = blockIdx.x * static_cast<int64_t>(kVecBS) + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * kVecBS;
+  const bool packed = aligned16(x, p, r);
+  const int64_t npk = packed ? n / N : 0; // 16-byte packs
+  Pack16<X> xa{}, pa{}, ra{};
+  auto load = [&](int64_t q) {
+    xa = ld16<true>(x + q * N), pa = ld16(p + q * N);
+    ra = ld16<kStreamLastRead<X>>(r + q * N);
+  };
+  if (gid < npk)
+    load(gid);
+  X alpha, beta;
+  coefficients(alpha, beta);
+  for (int64_t q = gid; q < npk; q += stride)
+  {
+    if (q != gid)
+      load(q);
+#pragma unroll
+    for (int e = 0; e < N; ++e)
+    {
+      const X pi = pa.v[e];
+      xa.v[e] = xa.v[e] + alpha * pi;
+      pa.v[e] = pi * beta + ra.v[e];
+    }
+    st16<true>(x + q * N, xa);
+    st16(p + q * N, pa);
+  }
+  for (int64_t i = npk * N + gid; i < n; i += stride)
+  {
+    const X pi = p[i];
+    __builtin_nontemporal_store(ld_stream<true>(x + i) + alpha * pi, x + i);
+    p[i] = pi * beta + ld_stream<kStreamLastRead<X>>(r + i);
+  }
+}
+
+// The same as a kernel: runs iff this iteration completed its residual update (also
+// on the iteration that stops).
 template <typename X, typename Acc>
 __global__ __launch_bounds__(kVecBS) void cg_update_xp(int64_t n, X* __restrict__ x,
                                                        X* __restrict__ p,
@@ -1175,37 +1228,10 @@ __global__ __launch_bounds__(kVecBS) void cg_update_xp(int64_t n, X* __restrict_
   (void)it;
   if (!st->xp_pending)
     return;
-  const X alpha = static_cast<X>(st->alpha);
-  const X beta = static_cast<X>(st->beta);
-  constexpr int N = Pack16<X>::N;
-  const int64_t gid = blockIdx.x * static_cast<int64_t>(kVecBS) + threadIdx.x;
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kVecBS;
-  int64_t done = 0; // elements covered by the 16-byte passes
-  if (aligned16(x, p, r))
-  {
-    const int64_t npk = n / N;
-    for (int64_t q = gid; q < npk; q += stride)
-    {
-      Pack16<X> xa = ld16<true>(x + q * N), pa = ld16(p + q * N);
-      const Pack16<X> ra = ld16<kStreamLastRead<X>>(r + q * N);
-#pragma unroll
-      for (int e = 0; e < N; ++e)
-      {
-        const X pi = pa.v[e];
-        xa.v[e] = xa.v[e] + alpha * pi;
-        pa.v[e] = pi * beta + ra.v[e];
-      }
-      st16<true>(x + q * N, xa);
-      st16(p + q * N, pa);
-    }
-    done = npk * N;
-  }
-  for (int64_t i = done + gid; i < n; i += stride)
-  {
-    const X pi = p[i];
-    __builtin_nontemporal_store(ld_stream<true>(x + i) + alpha * pi, x + i);
-    p[i] = pi * beta + ld_stream<kStreamLastRead<X>>(r + i);
-  }
+  update_xp<X>(n, x, p, r, [&](X& alpha, X& beta) {
+    alpha = static_cast<X>(st->alpha);
+    beta = static_cast<X>(st->beta);
+  });
 }
 
 } // namespace spmvx
