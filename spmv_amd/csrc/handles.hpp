@@ -162,6 +162,11 @@ int default_variant(int32_t dtype);
 // The same for a pattern: small FP64 matrices get small row blocks.
 int plain_variant(const Pattern& P, int32_t dtype);
 
+// Whether csr_wave runs the products of complex values whose variant is `var`: the
+// default one, where every row has a mask over the list of column offsets (builds
+// the analysis).
+bool complex_wave(Pattern& P, int32_t dtype, int var);
+
 // Stored entries and rows per row block of the CSR kernel of variant `var`:
 // csr_wave's where that kernel runs the variant.
 inline std::pair<int, int> variant_blocking(Pattern& P, int var)

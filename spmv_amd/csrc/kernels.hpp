@@ -500,7 +500,8 @@ __global__ __launch_bounds__(BS) void csr_stream(
 // non-temporal matrix loads, threads per workgroup (= rows per block at
 // most), short column indices}.  Variants 0-4 also take complex values.
 // Variants 8, 10 and 11, the 16-bit kernels that the matrices get by default,
-// run csr_wave instead where the matrix's rows suit it (wave_class).
+// run csr_wave instead where the matrix's rows suit it (wave_class); so do the
+// default variants of complex values (complex_wave).
 struct SpmvVariant
 {
   int chunk;
@@ -605,7 +606,7 @@ int64_t launch_csr_stream(int var, const CsrView& M, hipStream_t s, const V* val
 {
   if (M.nblocks <= 0)
     return 0;
-  if constexpr (!kIsComplex<V>)
+  if constexpr (!kIsComplex<V> || MODE == kPlain)
     if (M.wave >= 0)
     {
       launch_csr_wave<V, X, Acc, MODE>(M, s, val, x, y, b, partials, st, it, ev0, ev1);

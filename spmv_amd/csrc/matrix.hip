@@ -566,12 +566,37 @@ int plain_variant(const Pattern& P, int32_t dtype)
   return small_blocks_suit(P, dtype) ? 4 : default_variant(dtype);
 }
 
+// csr_wave reads the masks alone for complex values: its variant only names the row
+// blocks, which all of its variants share.
+constexpr int kWaveVariant = 11;
+
+// Blocks without masks (and the 16-bit indices they would need) are left to csr_stream:
+// stencils and their transposes, which complex fields live on, have masks throughout.
+// Single products from 300 thousand rows on, csr_stream and csr_wave, us: complex
+// FP64, bands of 3 to 27 entries 5.5 to 35 and 5.0 to 26, complex FP32 5.1 to 20 and
+// 5.3 to 14; on fewer rows both are bound by the call (7-point 30x30x20: 5.3 and 5.4).
+bool complex_wave(Pattern& P, int32_t dtype, int var)
+{
+  // (32-bit byte offsets into x: build_masks allows for 8 bytes per entry)
+  if (!is_complex(dtype) || forced_variant() >= 0 || var != default_variant(dtype)
+      || (dtype == SPMVX_C64 && std::max(P.nrows, P.ncols) > (int64_t(1) << 28) - 16)
+      || P.wave_class() < 0)
+    return false;
+  P.build_masks(variant_blocks(P, kWaveVariant));
+  return P.masked && P.all_masked;
+}
+
 int matrix_default_variant(spmvx_matrix_s* A)
 {
   Pattern& P = *A->pat;
   const int base = plain_variant(P, A->dtype);
-  if (forced_variant() >= 0 || is_complex(A->dtype))
+  if (forced_variant() >= 0)
     return base;
+  if (is_complex(A->dtype))
+  {
+    (void)complex_wave(P, A->dtype, base); // built here, not first in a product
+    return base;
+  }
   // the short-index kernel for the dtype when the matrix fits it (the
   // analysis of the inspector, Matrix.cpp:43); where the rows suit it, those
   // whose products csr_wave runs.  Otherwise FP64 the 16-bit counterpart of
@@ -773,7 +798,9 @@ template <typename V, typename X, typename Acc>
 void launch_plain(int var, Pattern& P, const void* vals, const void* x, void* y, hipStream_t s,
                   int32_t long_par, hipEvent_t ev0, hipEvent_t ev1)
 {
-  const CsrView M = csr_view(P, var, sizeof(V));
+  const bool cw = kIsComplex<V> && complex_wave(P, sizeof(V) == 16 ? SPMVX_C64 : SPMVX_C32, var);
+  const CsrView M = cw ? make_view(P, &variant_blocks(P, kWaveVariant), kWaveVariant, sizeof(V))
+                       : csr_view(P, var, sizeof(V));
   launch_csr_stream<V, X, Acc, kPlain>(var, M, s, static_cast<const V*>(vals),
                                        static_cast<const X*>(x), static_cast<X*>(y), nullptr,
                                        nullptr, nullptr, 0, long_par, ev0, ev1);
@@ -1151,10 +1178,13 @@ int spmvx_matrix_get_kernel(spmvx_matrix A, int32_t* variant, char* name, int32_
       else
       {
         const SpmvVariant& k = kVariants[v];
-        const int c = variant_wave(v) ? A->pat->wave_class() : -1;
+        const bool cw = complex_wave(*A->pat, A->dtype, v);
+        const int c = cw || variant_wave(v) ? A->pat->wave_class() : -1;
         if (c >= 0)
           d = "csr_wave (one wavefront per 64 rows, " + std::to_string(kWaveClasses[c].kr)
-              + (A->pat->masked ? " column offsets and a mask per row, else " : " gathers at once, ");
+              + (cw               ? " column offsets and a mask per row"
+                 : A->pat->masked ? " column offsets and a mask per row, else "
+                                  : " gathers at once, ");
         else
           d = std::string("csr_stream (") + std::to_string(k.bs) + " threads, chunk "
               + std::to_string(k.chunk) + ", vec " + std::to_string(k.vec) + ", unroll "

@@ -39,9 +39,13 @@ namespace spmvx
 // best then (wave_plan).  burst = 0: every block's results are stored at once,
 // for matrices with too few blocks to fill bursts.
 //
+// Complex values: only matrices whose blocks all have masks (complex_wave).
+//
 // Bound by HBM.  27-point 160^3, FP64: csr_stream 222 us, here with indices 176,
 // with masks 150 (0.97 GB: 6.5 TB/s, a streaming read runs at 7.0).  7-point 256^3:
-// FP64 313 to 218 us, FP32 188 to 117, BF16 168 to 89.
+// FP64 313 to 218 us, FP32 188 to 117, BF16 168 to 89.  Complex FP64, csr_stream's 129
+// to 90 us (7-point 160^3), 9.0 to 6.8 (63x65x61), 123 to 67 (27-point 100^3); complex
+// FP32, 7-point 160^3, 83 to 51.
 constexpr int kWaveRows = 64;
 
 // 1 KiB LDS loads (64 lanes of 16 bytes) that hold n entries of es bytes.
@@ -74,29 +78,31 @@ __device__ __forceinline__ void lds_filled()
 }
 
 // Sizes of csr_wave: E entries staged per block, KR entries of a row gathered
-// at once, and the wavefronts per CU of a streaming product (B > 0) for 8-, 4-
-// and 2-byte values.  KR are the widths of the 3-, 5-, 7-, 9- and 27-point
+// at once, and the wavefronts per CU of a streaming product (B > 0) for 16-, 8-,
+// 4- and 2-byte values.  KR are the widths of the 3-, 5-, 7-, 9- and 27-point
 // operators and one between; E holds 64 such rows, up to 7 entries before the
 // block (aligned loads) and KR entries read past the last row.
 // Wavefronts per CU: the best of the counts tried, matrices of the KR's width
 // with row masks in HBM (FP64 7-point 256^3 6 / 7 / 9 wavefronts: 223 / 218 / 235 us,
 // 27-point 160^3 3 / 4 / 5: 152 / 149 / 163; FP32 7-point 10 / 12 / 16: 123 / 117 /
-// 127, 27-point 6 / 8 / 10: 83 / 82 / 85).  Enough loads must be in flight, and
+// 127, 27-point 6 / 8 / 10: 83 / 82 / 85; complex FP64 7-point 160^3 4 / 5 / 6: 92.2 /
+// 90.5 / 91.7, 27-point 100^3 2 / 3 / 4: 73 / 67 / 69; complex FP32 stays within 2% of
+// its best with FP64's).  Enough loads must be in flight, and
 // each further stream costs HBM efficiency: wide rows (more bytes and gathers
 // per wavefront) want fewer.
 struct WaveClass
 {
-  int e, kr, per_cu8, per_cu4, per_cu2;
+  int e, kr, per_cu16, per_cu8, per_cu4, per_cu2;
 };
 #define SPMVX_WAVE_CLASSES(X)                                                                \
-  X(0, 256, 3, 12, 20, 20)                                                                   \
-  X(1, 384, 5, 9, 16, 20)                                                                    \
-  X(2, 512, 7, 7, 12, 16)                                                                    \
-  X(3, 640, 9, 7, 12, 12)                                                                    \
-  X(4, 1024, 15, 4, 8, 12)                                                                   \
-  X(5, 1792, 27, 4, 8, 12)
+  X(0, 256, 3, 10, 12, 20, 20)                                                              \
+  X(1, 384, 5, 7, 9, 16, 20)                                                                \
+  X(2, 512, 7, 5, 7, 12, 16)                                                                \
+  X(3, 640, 9, 4, 7, 12, 12)                                                                \
+  X(4, 1024, 15, 3, 4, 8, 12)                                                               \
+  X(5, 1792, 27, 3, 4, 8, 12)
 constexpr int kNumWaveClasses = 6;
-#define SPMVX_WAVE_ENTRY(i, E, K, W8, W4, W2) {E, K, W8, W4, W2},
+#define SPMVX_WAVE_ENTRY(i, E, K, W16, W8, W4, W2) {E, K, W16, W8, W4, W2},
 constexpr WaveClass kWaveClasses[kNumWaveClasses] = {SPMVX_WAVE_CLASSES(SPMVX_WAVE_ENTRY)};
 #undef SPMVX_WAVE_ENTRY
 // Stored entries that a block of a class may hold.
@@ -141,10 +147,25 @@ __device__ __forceinline__ X ld_buffer(const X* x, uint32_t bytes, uint32_t off)
 {
   __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<X*>(x), 0, static_cast<int32_t>(bytes), 0x00020000);
-  if constexpr (sizeof(X) == 8)
+  if constexpr (sizeof(X) == 16)
+    return __builtin_bit_cast(X, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  else if constexpr (sizeof(X) == 8)
     return __builtin_bit_cast(X, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
   else
     return __builtin_bit_cast(X, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
+}
+
+// A non-temporal store.
+template <typename T>
+__device__ __forceinline__ void store_streamed(T* p, T v)
+{
+  __builtin_nontemporal_store(v, p);
+}
+template <typename T>
+__device__ __forceinline__ void store_streamed(cplx<T>* p, cplx<T> v)
+{
+  store_streamed(&p->re, v.re);
+  store_streamed(&p->im, v.im);
 }
 
 // Sum of v (< 2^BITS) over the lanes below this one.
@@ -180,6 +201,7 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
     return;
   constexpr int NV = wave_loads(E, sizeof(V)), NX = wave_loads(E, 2);
   constexpr int AL = 8; // entries: 16 bytes of indices
+  constexpr bool ALL = kIsComplex<V>; // every block has masks (complex_wave)
   extern __shared__ __align__(16) char buf[];
   const lds_ptr fill_at = (lds_ptr)buf;
   const V* lval = reinterpret_cast<const V*>(buf);
@@ -224,7 +246,7 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
     auto fill = [&](int32_t a, int32_t e, int32_t masked) {
       const int32_t kb = a & ~(AL - 1);
       const int32_t n = (e - kb + AL - 1) & ~(AL - 1);
-      if (!HM || !masked)
+      if (!ALL && (!HM || !masked))
         lds_fill<NX, kLoadStream>(reinterpret_cast<const char*>(col16 + kb), n * 2, fill_at + at.col_at);
       const char* g = reinterpret_cast<const char*>(val + kb);
       const int32_t bytes = n * static_cast<int32_t>(sizeof(V));
@@ -236,11 +258,14 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
     int32_t of[KR]; // the list of column offsets, as byte offsets into x
 #pragma unroll
     for (int k = 0; k < KR; ++k)
-      of[k] = HM ? offs[k] * static_cast<int32_t>(sizeof(X)) : 0;
+      of[k] = HM ? static_cast<int32_t>(static_cast<uint32_t>(offs[k])
+                                        * static_cast<uint32_t>(sizeof(X)))
+                 : 0;
     kind = blocks[bi].x;
     k0 = blocks[bi].y;
     k1 = blocks[bi + 1].y;
-    w = wbase[bi];
+    if constexpr (!ALL)
+      w = wbase[bi];
     load_rows(bi, ra, re, xr);
     fill(k0, k1, kind);
 
@@ -280,7 +305,7 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
           {
             const int32_t row = (kfirst + t * nw) * kWaveRows + lane;
             if (row < nrows)
-              __builtin_nontemporal_store(kept[t * kWaveRows + lane], y + row);
+              store_streamed(y + row, kept[t * kWaveRows + lane]);
           }
         nkept = 0;
       }
@@ -297,7 +322,8 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
         nkind = blocks[nb].x;
         n0 = blocks[nb].y;
         n1 = blocks[nb + 1].y;
-        nwb = wbase[nb];
+        if constexpr (!ALL)
+          nwb = wbase[nb];
       }
       // row's first entry in LDS and its length
       int32_t pos, len;
@@ -424,7 +450,9 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
       xr = nxr;
     };
     auto step = [&](auto refill, int32_t nb) {
-      if (HM && kind)
+      if constexpr (ALL)
+        block(refill, std::true_type{}, nb);
+      else if (HM && kind)
         block(refill, std::bool_constant<HM != 0>{}, nb);
       else
         block(refill, std::false_type{}, nb);
@@ -457,8 +485,10 @@ constexpr int64_t kWaveMaxGrid = 8192; // 32 wavefronts on each of 256 CUs
 inline WavePlan wave_plan(int c, int vbytes, bool cols, int64_t nblocks, int ncu)
 {
   const WaveClass& k = kWaveClasses[c];
-  const int xbytes = vbytes == 8 ? 8 : 4;
-  const int per = vbytes == 8 ? k.per_cu8 : (vbytes == 4 ? k.per_cu4 : k.per_cu2);
+  const int xbytes = vbytes >= 8 ? vbytes : 4;
+  const int per = vbytes == 16 ? k.per_cu16
+                  : vbytes == 8 ? k.per_cu8
+                                : (vbytes == 4 ? k.per_cu4 : k.per_cu2);
   const int64_t stream = static_cast<int64_t>(ncu) * per;
   if (nblocks >= 8 * stream)
   {
@@ -512,8 +542,10 @@ void launch_csr_wave(const CsrView& M, hipStream_t s, const V* val, const X* x, 
   };
   using std::integral_constant;
   auto kinds = [&](auto e, auto kr) {
-    if (hm)
+    if (kIsComplex<V> || hm)
       go(integral_constant<int, 2>{}, integral_constant<int, 1>{}, e, kr);
+    else if constexpr (kIsComplex<V>)
+      return;
     else if (M.short_kind == 1)
       go(integral_constant<int, 1>{}, integral_constant<int, 0>{}, e, kr);
     else
@@ -521,7 +553,7 @@ void launch_csr_wave(const CsrView& M, hipStream_t s, const V* val, const X* x, 
   };
   switch (M.wave)
   {
-#define SPMVX_WAVE_CASE(i, EE, K, W8, W4, W2)                                                  \
+#define SPMVX_WAVE_CASE(i, EE, K, W16, W8, W4, W2)                                             \
   case i: kinds(integral_constant<int, EE>{}, integral_constant<int, K>{}); break;
     SPMVX_WAVE_CLASSES(SPMVX_WAVE_CASE)
 #undef SPMVX_WAVE_CASE
