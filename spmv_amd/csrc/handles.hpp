@@ -137,6 +137,7 @@ struct Pattern
   // first use
   int wave_class();
   int wave = -2;          // -2: not analysed yet
+  bool transposed = false; // of a transposed copy (products alone use it)
   int ncu = 0;            // compute units of the device
   int64_t widest_row = 0; // a row of the largest length
   int32_t longest = 0;    // entries of the longest row
@@ -159,7 +160,7 @@ std::vector<int2> row_blocks(const int32_t* rowptr, int64_t nrows, int64_t max_n
 
 // Default kernel variant of a value type (overridable with SPMVX_SPMV_VARIANT).
 int default_variant(int32_t dtype);
-// The same for a pattern: small FP64 matrices get small row blocks.
+// The same for a pattern: small FP64 matrices and transposed ones get small row blocks.
 int plain_variant(const Pattern& P, int32_t dtype);
 
 // Whether csr_wave runs the products of complex values whose variant is `var`: the

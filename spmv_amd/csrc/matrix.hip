@@ -561,9 +561,16 @@ bool small_blocks_suit(const Pattern& P, int32_t dtype)
 }
 } // namespace
 
+// Transposed FP64 products from 32-bit indices get the small blocks at any size: their
+// columns are spread (those of stencils fit 16 bits), and more blocks keep more gathers
+// in flight.  us with 8192 and 2048 entries a block: transposed assembly maps, 6.5
+// million entries 28.1 and 25.0, 8.4 million 36.9 and 31.6, 18 million 65.9 and 62.9, 72
+// million 298 and 291; random rows, 4.8 million 40.9 and 36.4, 38 million 600 and 578.
+// A matrix's own product keeps 8192 above the limit: CG sums its blocks' partials.
 int plain_variant(const Pattern& P, int32_t dtype)
 {
-  return small_blocks_suit(P, dtype) ? 4 : default_variant(dtype);
+  const bool spread = P.transposed && dtype == SPMVX_F64 && forced_variant() < 0;
+  return spread || small_blocks_suit(P, dtype) ? 4 : default_variant(dtype);
 }
 
 // csr_wave reads the masks alone for complex values: its variant only names the row
@@ -586,15 +593,15 @@ bool complex_wave(Pattern& P, int32_t dtype, int var)
   return P.masked && P.all_masked;
 }
 
-int matrix_default_variant(spmvx_matrix_s* A)
+// Default variant of a pattern (whatever it needs is built here, not first in a product).
+int pattern_default_variant(Pattern& P, int32_t dtype)
 {
-  Pattern& P = *A->pat;
-  const int base = plain_variant(P, A->dtype);
+  const int base = plain_variant(P, dtype);
   if (forced_variant() >= 0)
     return base;
-  if (is_complex(A->dtype))
+  if (is_complex(dtype))
   {
-    (void)complex_wave(P, A->dtype, base); // built here, not first in a product
+    (void)complex_wave(P, dtype, base);
     return base;
   }
   // the short-index kernel for the dtype when the matrix fits it (the
@@ -604,13 +611,18 @@ int matrix_default_variant(spmvx_matrix_s* A)
   // 16-byte index loads (vec 8: FP32 bands of 20 million entries 65.5 us, vec 4 x
   // unroll 2 74.8, 2048-entry blocks 85.4; BF16 57, 61 and 79)
   const bool wave = P.wave_class() >= 0;
-  const int sv = A->dtype == SPMVX_F64 ? (!wave && small_blocks_suit(P, A->dtype) ? 9 : 8)
-                 : A->dtype == SPMVX_F32 && wave ? 11
+  const int sv = dtype == SPMVX_F64 ? (!wave && small_blocks_suit(P, dtype) ? 9 : 8)
+                 : dtype == SPMVX_F32 && wave ? 11
                                                  : 10;
   if (P.nnz > 0 && fits_short(P, sv))
     return sv;
   (void)variant_blocks(P, base);
   return base;
+}
+
+int matrix_default_variant(spmvx_matrix_s* A)
+{
+  return pattern_default_variant(*A->pat, A->dtype);
 }
 
 namespace
@@ -963,12 +975,15 @@ namespace
 {
 
 // CSR kernel variant of the transposed product: the matrix's, unless it is
-// the sliced layout or a 16-bit-index kernel that the transposed pattern
-// does not fit (then the dtype's 32-bit default).
+// the sliced layout (then the transposed pattern's default), the 32-bit default or a
+// 16-bit-index kernel that the transposed pattern does not fit (then the transposed
+// pattern's 32-bit default).
 int transposed_variant(spmvx_matrix_s* A)
 {
   const int v = A->variant;
-  if (v == kSlicedVariant || (variant_short(v) && !fits_short(*A->tpat, v)))
+  if (v == kSlicedVariant)
+    return pattern_default_variant(*A->tpat, A->dtype);
+  if (variant_short(v) ? !fits_short(*A->tpat, v) : v == plain_variant(*A->pat, A->dtype))
     return plain_variant(*A->tpat, A->dtype);
   return v;
 }

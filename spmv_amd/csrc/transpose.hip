@@ -146,6 +146,7 @@ void build_transpose(spmvx_matrix_s* A, hipStream_t s)
                              sizeof(int32_t) * static_cast<size_t>(ncols + 1),
                              hipMemcpyDeviceToHost, s));
   SPMVX_HIP(hipStreamSynchronize(s));
+  T->transposed = true;
   const int var = plain_variant(*T, A->dtype);
   if (!complex_wave(*T, A->dtype, var))
     (void)variant_blocks(*T, var);
