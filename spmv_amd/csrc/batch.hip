@@ -749,6 +749,7 @@ struct spmvx_batch_s
   // 126, 8192 81, 4096 66, 2048 66 ms (an exchange costs about 3 us, and the largest
   // systems are the tail of the schedule).
   int32_t rows_per_member = 4096;
+  bool members_set = false; // by spmvx_batch_set_config
   int grid = 0;
   // captured graph and the arguments it was captured with
   hipGraphExec_t exec = nullptr;
@@ -922,7 +923,11 @@ void build_plan(spmvx_batch_s* B, int capacity)
           lanes_for(rows > 0 ? static_cast<int>((nz + rows - 1) / rows) : 1));
     }
     int64_t w = 1;
-    if (B->rows_per_member > 0)
+    if (B->rows_per_member > 0 && B->members_set)
+      // the caller's choice, up to wmax (256 systems of 1000 to 200000 rows, 4096 rows a
+      // member: 453 ms, 530 with the bound below)
+      w = div_up(rows, B->rows_per_member);
+    else if (B->rows_per_member > 0)
       // Members of less than kWideMember rows only in teams of up to kSmallTeam: a
       // launch holds at most one gathering team per queue, 8 x 7 workgroups, so that
       // launches on 4 streams (the hardware queues of a process) cannot fill the 256
@@ -1163,11 +1168,13 @@ int spmvx_batch_set_config(spmvx_batch B, int32_t block, int32_t lanes_per_row,
                       || lanes_per_row == 4 || lanes_per_row == 8 || lanes_per_row == 16,
                   "lanes_per_row must be 0 (per system), 1, 2, 4, 8 or 16");
     SPMVX_REQUIRE(rows_per_member >= 0, "rows_per_member must be >= 0");
-    if (block != B->block || lanes_per_row != B->g_policy || rows_per_member != B->rows_per_member)
+    if (block != B->block || lanes_per_row != B->g_policy || rows_per_member != B->rows_per_member
+        || !B->members_set)
     {
       B->block = block;
       B->g_policy = lanes_per_row;
       B->rows_per_member = rows_per_member;
+      B->members_set = true;
       B->plan_dirty = true;
       drop_graph(B);
     }

@@ -70,3 +70,17 @@ def test_wide_members_beyond_a_small_team(rows):
     x, _ = B.solve(torch.from_numpy(b).cuda(), max_its=500, rtol=1e-5)
     assert residuals(systems[0], b[:rows], x.cpu().numpy()[:rows]).max() <= 1e-5 * (1 + 1e-9)
     assert B.config()["slots"] == max(8, -(-rows // 16384)) + 1
+
+
+@pytest.mark.parametrize("rows", [40000, 131073])
+def test_chosen_members_are_not_widened(rows):
+    """Rows per member set by the caller: teams of as many members as they give, up to a
+    sixteenth of the workgroups."""
+    systems = [Banded(rows, 2), Banded(50, 2)]
+    B = S.Batch(systems, nrhs=4)
+    B.set_config(1024, 0, 4096)
+    b = np.random.default_rng(6).uniform(-1, 1, (B.nrows, 4)).astype(np.float32)
+    x, _ = B.solve(torch.from_numpy(b).cuda(), max_its=500, rtol=1e-5)
+    assert residuals(systems[0], b[:rows], x.cpu().numpy()[:rows]).max() <= 1e-5 * (1 + 1e-9)
+    c = B.config()
+    assert c["slots"] == min(c["grid"] // 16, -(-rows // 4096)) + 1
