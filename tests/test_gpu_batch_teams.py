@@ -75,12 +75,12 @@ def test_wide_members_beyond_a_small_team(rows):
 @pytest.mark.parametrize("rows", [40000, 131073])
 def test_chosen_members_are_not_widened(rows):
     """Rows per member set by the caller: teams of as many members as they give, up to a
-    sixteenth of the workgroups."""
+    sixteenth of the CUs (one workgroup of 1024 threads each)."""
     systems = [Banded(rows, 2), Banded(50, 2)]
     B = S.Batch(systems, nrhs=4)
     B.set_config(1024, 0, 4096)
     b = np.random.default_rng(6).uniform(-1, 1, (B.nrows, 4)).astype(np.float32)
     x, _ = B.solve(torch.from_numpy(b).cuda(), max_its=500, rtol=1e-5)
     assert residuals(systems[0], b[:rows], x.cpu().numpy()[:rows]).max() <= 1e-5 * (1 + 1e-9)
-    c = B.config()
-    assert c["slots"] == min(c["grid"] // 16, -(-rows // 4096)) + 1
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert B.config()["slots"] == min(cus // 16, -(-rows // 4096)) + 1
