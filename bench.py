@@ -617,7 +617,7 @@ def main():
                      "hbm_GBps_measured": (round(traffic / (spmv_ms * 1e-3) / 1e9, 1)
                                            if traffic else None),
                      "note": ("achieved = the algorithmic CSR bytes (4-byte column indices) "
-                              "per product / kernel time; a kernel reading 16-bit column "
+                              "per product / kernel time; a kernel reading row masks or 16-bit "
                               "indices moves fewer bytes (traffic), so hbm_GBps_measured is "
                               "the bandwidth it actually draws")},
         "csr_int32_indices": int32_kernel,
