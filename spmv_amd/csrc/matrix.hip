@@ -1152,6 +1152,8 @@ int spmvx_matrix_set_kernel(spmvx_matrix A, int32_t variant)
     else
       (void)csr_view(*A->pat, v, dtype_size(A->dtype)); // row blocks (and short indices) built here
     A->variant = v;
+    if (A->tpat) // and those of the transposed copy, so that its products can be captured
+      (void)csr_view(*A->tpat, transposed_variant(A), dtype_size(A->dtype));
   });
 }
 
