@@ -56,18 +56,21 @@ constexpr int kLoadKeep = 0, kLoadStream = 2;
 
 // Requests `bytes` bytes (a multiple of 16, at most N KiB) from g (16-byte
 // aligned) into LDS; lanes past the end are out of the buffer's range and read
-// nothing.  The caller waits (lds_filled): the compiler does not order LDS
-// reads after these loads.
+// nothing.  A load's whole distance from g is in the lane's offset: the scalar
+// offset of a buffer load takes no part in the range check, and with i KiB there
+// the last loads of a short block would read up to N KiB past the arrays.  The caller
+// waits (lds_filled): the compiler does not order LDS reads after these loads.
 typedef __attribute__((address_space(3))) char* lds_ptr;
 template <int N, int AUX>
 __device__ __forceinline__ void lds_fill(const char* g, int32_t bytes, lds_ptr lds)
 {
   __amdgpu_buffer_rsrc_t r =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(g), 0, bytes, 0x00020000);
-  const int32_t off = static_cast<int32_t>(threadIdx.x) * 16;
+  int32_t off = static_cast<int32_t>(threadIdx.x) * 16;
+  asm volatile("" : "+v"(off)); // (the sums below are formed here, not kept in N registers)
 #pragma unroll
   for (int i = 0; i < N; ++i)
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds + i * 1024, 16, off, i * 1024, 0, AUX);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, lds + i * 1024, 16, off + i * 1024, 0, 0, AUX);
 }
 
 // Waits for every vector memory operation of this wavefront (the loads of
