@@ -160,15 +160,54 @@ __device__ __forceinline__ X ld_buffer(const X* x, uint32_t bytes, uint32_t off)
 
 // A non-temporal store.
 template <typename T>
-__device__ __forceinline__ void store_streamed(T* p, T v)
+__host__ __device__ __forceinline__ void store_streamed(T* p, T v)
 {
   __builtin_nontemporal_store(v, p);
 }
 template <typename T>
-__device__ __forceinline__ void store_streamed(cplx<T>* p, cplx<T> v)
+__host__ __device__ __forceinline__ void store_streamed(cplx<T>* p, cplx<T> v)
 {
   store_streamed(&p->re, v.re);
   store_streamed(&p->im, v.im);
+}
+
+// This lane's share of storing the results of nkept blocks (first, first + nw, ...) kept
+// in LDS, kWaveRows of each: 16 bytes at a time where y allows it.  Lanes past the last
+// kept block read nothing: a burst need not fill the blocks of one store.
+template <typename X>
+__host__ __device__ __forceinline__ void store_burst(const X* kept, int32_t nkept, int32_t first,
+                                                     int32_t nw, int32_t nrows, X* y, int lane)
+{
+  if ((reinterpret_cast<uintptr_t>(y) & 15) == 0)
+  {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    constexpr int N = 16 / sizeof(X), LPB = kWaveRows / N; // per lane; lanes per block
+    const int32_t step = kWaveRows / LPB;                  // blocks per store
+#pragma unroll 4
+    for (int32_t t0 = 0; t0 < nkept; t0 += step)
+    {
+      const int32_t t = t0 + lane / LPB;
+      if (t < nkept)
+      {
+        const X* k = kept + t0 * kWaveRows + lane * N;
+        const int32_t row = (first + t * nw) * kWaveRows + (lane % LPB) * N;
+        if (row + N <= nrows)
+          __builtin_nontemporal_store(*reinterpret_cast<const u4*>(k),
+                                      reinterpret_cast<u4*>(y + row));
+        else
+          for (int i = 0; row + i < nrows; ++i)
+            y[row + i] = k[i];
+      }
+    }
+  }
+  else
+#pragma unroll 1
+    for (int32_t t = 0; t < nkept; ++t)
+    {
+      const int32_t row = (first + t * nw) * kWaveRows + lane;
+      if (row < nrows)
+        store_streamed(y + row, kept[t * kWaveRows + lane]);
+    }
 }
 
 // Sum of v (< 2^BITS) over the lanes below this one.
@@ -281,35 +320,7 @@ void csr_wave(const int32_t* __restrict__ rows, const int2* __restrict__ blocks,
     auto store_kept = [&]() {
       if (burst > 0)
       {
-        if ((reinterpret_cast<uintptr_t>(y) & 15) == 0)
-        {
-          typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-          constexpr int N = 16 / sizeof(X), LPB = kWaveRows / N; // per lane; lanes per block
-          const int32_t step = kWaveRows / LPB;                  // blocks per store
-#pragma unroll 4
-          for (int32_t t0 = 0; t0 < nkept; t0 += step)
-          {
-            const int32_t t = t0 + lane / LPB;
-            const int32_t row = (kfirst + t * nw) * kWaveRows + (lane % LPB) * N;
-            const u4 v = *reinterpret_cast<const u4*>(kept + t0 * kWaveRows + lane * N);
-            if (t < nkept)
-            {
-              if (row + N <= nrows)
-                __builtin_nontemporal_store(v, reinterpret_cast<u4*>(y + row));
-              else
-                for (int i = 0; row + i < nrows; ++i)
-                  y[row + i] = kept[t0 * kWaveRows + lane * N + i];
-            }
-          }
-        }
-        else
-#pragma unroll 1
-          for (int32_t t = 0; t < nkept; ++t)
-          {
-            const int32_t row = (kfirst + t * nw) * kWaveRows + lane;
-            if (row < nrows)
-              store_streamed(y + row, kept[t * kWaveRows + lane]);
-          }
+        store_burst(kept, nkept, kfirst, nw, nrows, y, lane);
         nkept = 0;
       }
       else if (yrow >= 0)
