@@ -398,8 +398,11 @@ int spmvx_batch_set_config(spmvx_batch B, int32_t block, int32_t lanes_per_row,
  * recursive residual, at most 4 times per solve, so the returned x meets
  * ||b - A x|| <= rtol ||b|| and not only the FP32 recursion.
  * its_host (may be NULL): nsys*nrhs iteration counts (counted on across
- * restarts).  The stream is synchronised; a timed-out team wait is reported
- * as SPMVX_ERR_STATE (results invalid).
+ * restarts; -1 for a system that the solve did not finish, which only a failed
+ * solve has).  The stream is synchronised; a team wait that runs out
+ * (after 2^22 polls, a few seconds; SPMVX_BATCH_SPIN_LIMIT at creation sets
+ * another number) ends the solve and is reported as SPMVX_ERR_STATE (results
+ * invalid; the batch can be solved again).
  */
 int spmvx_batch_solve(spmvx_batch B, const float* b_dev, float* x_dev, int32_t max_its,
                       double rtol, int32_t* its_host, spmvx_stream stream);

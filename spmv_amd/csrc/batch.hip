@@ -261,13 +261,39 @@ __device__ __forceinline__ VecN<NRHS> batch_spmv(const int32_t* __restrict__ row
   return pdy;
 }
 
-// Bounded spin: a team barrier gives up (and flags the solve as failed)
-// after about this many polls (a few seconds) instead of waiting forever; a
-// legitimate wait lasts at most one team member's solve of another system.
+// Bounded waits: a wait of a team gives up after this many polls (a few seconds;
+// SPMVX_BATCH_SPIN_LIMIT at creation sets another number) instead of going on
+// forever; a legitimate one lasts at most one team member's solve of another system.
+// A member that gives up flags the solve as failed (err) and leaves the system.  A
+// peer never sees the words that the member would have written, and would run
+// into the limit at every further exchange; so whoever waits for longer than
+// kSpinFast polls reads the flag too and leaves, and no workgroup takes another
+// system once it is set: the grid drains about one limit after the first wait began.
 constexpr unsigned kSpinLimit = 1u << 22;
 // Polls without a pause (an exchange in step takes a few); longer waits, a team
 // still gathering members, leave the memory alone in between.
 constexpr unsigned kSpinFast = 64;
+
+// Failure handling of a solve: the flag all workgroups share, the limit, and this
+// workgroup's own note (LDS) that it leaves its system.
+struct TeamWaits
+{
+  int* err;
+  unsigned limit;
+  int* left;
+};
+
+// One unsuccessful poll: whether to stop waiting.
+__device__ __forceinline__ bool wait_over(unsigned& spins, const TeamWaits& w)
+{
+  if (spins++ >= w.limit)
+    atomicExch(w.err, 1);
+  else if (spins <= kSpinFast
+           || __hip_atomic_load(w.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+    return false;
+  *w.left = 1;
+  return true;
+}
 
 // Barrier among the W workgroups of one team (all of them are running: a
 // workgroup joins a team only by taking one of its slots from the queue).
@@ -277,8 +303,8 @@ constexpr unsigned kSpinFast = 64;
 // written before the barrier visible to every member (members may run on
 // different XCDs, whose L2s are not coherent with each other: the release
 // writes this XCD's L2 back, the acquire invalidates it; a full fence on
-// both sides would do each twice).
-__device__ __forceinline__ void team_barrier(unsigned* bar, unsigned target, int* err)
+// both sides would do each twice).  False (in all threads): leave the system.
+__device__ __forceinline__ bool team_barrier(unsigned* bar, unsigned target, const TeamWaits& w)
 {
   __syncthreads();
   if (threadIdx.x == 0)
@@ -289,30 +315,28 @@ __device__ __forceinline__ void team_barrier(unsigned* bar, unsigned target, int
     while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
     {
       __builtin_amdgcn_s_sleep(2);
-      if (++spins > kSpinLimit)
-      {
-        atomicExch(err, 1);
+      if (wait_over(spins, w))
         break;
-      }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
+  return *w.left == 0;
 }
 
 // Team-wide sum of per-thread values: the workgroup's sum goes to the member's
 // words of buffer seq & 1, every member's are polled until they carry seq (all
 // words zeroed before the launch), summed in member order.  The two buffers
 // alternate: a member writes sequence seq + 2 only after every member has written
-// seq + 1, that is, has read seq.
+// seq + 1, that is, has read seq.  False (in all threads): leave the system.
 template <int NRHS>
-__device__ __forceinline__ VecN<NRHS> team_total(VecN<NRHS> v, uint64_t* words, unsigned seq, int W,
-                                                 int m, int* err, float (*red)[16],
-                                                 float* total)
+__device__ __forceinline__ bool team_total(VecN<NRHS>& v, uint64_t* words, unsigned seq, int W,
+                                           int m, const TeamWaits& w, float (*red)[16],
+                                           float* total)
 {
   v = block_sum_n<NRHS>(v, red);
   if (W == 1)
-    return v;
+    return true;
   if (threadIdx.x < 64)
   {
     uint64_t* buf = words + static_cast<int64_t>(seq & 1u) * W * NRHS;
@@ -340,13 +364,8 @@ __device__ __forceinline__ VecN<NRHS> team_total(VecN<NRHS> v, uint64_t* words, 
           all = all && static_cast<unsigned>(q >> 32) == seq;
           o.v[j] = __uint_as_float(static_cast<uint32_t>(q));
         }
-        if (all)
+        if (all || wait_over(spins, w))
           wait = false;
-        else if (++spins > kSpinLimit)
-        {
-          atomicExch(err, 1);
-          wait = false;
-        }
         else if (spins > kSpinFast)
           __builtin_amdgcn_s_sleep(8);
       }
@@ -360,35 +379,37 @@ __device__ __forceinline__ VecN<NRHS> team_total(VecN<NRHS> v, uint64_t* words, 
     }
   }
   __syncthreads();
-  VecN<NRHS> t;
 #pragma unroll
   for (int j = 0; j < NRHS; ++j)
-    t.v[j] = total[j];
-  return t;
+    v.v[j] = total[j];
+  return *w.left == 0;
 }
 
 // Team-wide sum in double: member m stores its block sum in slot m of buffer
 // `which` (two alternate), then every member adds the W slots in member order.
+// False (in all threads): leave the system.
 template <int NRHS>
-__device__ __forceinline__ VecD<NRHS> team_sum_d(VecD<NRHS> v, double* tredd, int which, int W,
-                                                 int m, unsigned* bar, unsigned& nbar, int* err,
-                                                 double (*red)[16])
+__device__ __forceinline__ bool team_sum_d(VecD<NRHS>& v, double* tredd, int which, int W, int m,
+                                           unsigned* bar, unsigned& nbar, const TeamWaits& w,
+                                           double (*red)[16])
 {
   v = block_sum_d<NRHS>(v, red);
   if (W == 1)
-    return v;
+    return true;
   double* buf = tredd + static_cast<int64_t>(which) * W * NRHS;
   if (threadIdx.x == 0)
 #pragma unroll
     for (int j = 0; j < NRHS; ++j)
       buf[m * NRHS + j] = v.v[j];
-  team_barrier(bar, static_cast<unsigned>(W) * (++nbar), err);
+  if (!team_barrier(bar, static_cast<unsigned>(W) * (++nbar), w))
+    return false;
   VecD<NRHS> t{};
   for (int q = 0; q < W; ++q)
 #pragma unroll
     for (int j = 0; j < NRHS; ++j)
       t.v[j] += buf[q * NRHS + j];
-  return t;
+  v = t;
+  return true;
 }
 
 // Stores a row of p (or x) past this XCD's L2, so that members on other XCDs
@@ -412,7 +433,8 @@ __device__ __forceinline__ void stn_agent(float* p, const VecN<NRHS>& v)
 // Barrier of a team after stores past the L2 (stn_agent): they have completed
 // before the member's arrival (its waves wait for their stores at the first
 // workgroup barrier), and the caches are invalidated before any load behind it.
-__device__ __forceinline__ void team_publish(unsigned* bar, unsigned target, int* err)
+// False (in all threads): leave the system.
+__device__ __forceinline__ bool team_publish(unsigned* bar, unsigned target, const TeamWaits& w)
 {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();
@@ -422,17 +444,15 @@ __device__ __forceinline__ void team_publish(unsigned* bar, unsigned target, int
     unsigned spins = 0;
     while (__hip_atomic_load(bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target)
     {
-      if (++spins > kSpinLimit)
-      {
-        atomicExch(err, 1);
+      if (wait_over(spins, w))
         break;
-      }
       if (spins > kSpinFast)
         __builtin_amdgcn_s_sleep(8);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
+  return *w.left == 0;
 }
 
 // Index of the XCD (accelerator complex die) the calling wave runs on, from
@@ -457,9 +477,11 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
     const float* __restrict__ b, float* __restrict__ xu, float* __restrict__ xin,
     float* __restrict__ r, float* __restrict__ p, float* __restrict__ y, int32_t max_its,
     float rtol2, double rtol2d, int32_t* __restrict__ its_out, unsigned* queue, unsigned* bars,
-    double* tred_all, uint64_t* words_all, int* err)
+    double* tred_all, uint64_t* words_all, int* err, unsigned spin_limit)
 {
   __shared__ int2 job;
+  __shared__ int left;
+  const TeamWaits waits{err, spin_limit, &left};
   __shared__ float total[2][NRHS];
   __shared__ float red[NRHS][16];
   __shared__ double redd[NRHS][16];
@@ -473,6 +495,9 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
     if (threadIdx.x == 0)
     {
       int2 jbv = make_int2(-1, 0);
+      left = 0;
+      if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+        t = nq; // the solve has failed
       while (t < nq)
       {
         const int q = (home + t) % nq;
@@ -525,9 +550,11 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
 #pragma unroll
     for (int j = 0; j < NRHS; ++j)
       bb.v[j] = static_cast<double>(rr.v[j]);
-    if (W > 1)
-      team_publish(bar, static_cast<unsigned>(W) * (++nbar), err); // p complete
-    rr = team_total<NRHS>(rr, words, ++seq, W, m, err, red, total[seq & 1]);
+    if (W > 1 && !team_publish(bar, static_cast<unsigned>(W) * (++nbar), waits)) // p complete
+      continue;
+    ++seq;
+    if (!team_total<NRHS>(rr, words, seq, W, m, waits, red, total[seq & 1]))
+      continue;
     {
       VecD<NRHS> b2{};
       for (int32_t i = lo + static_cast<int32_t>(threadIdx.x); i < hi; i += blockDim.x)
@@ -537,7 +564,9 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
         for (int j = 0; j < NRHS; ++j)
           b2.v[j] += static_cast<double>(bi.v[j]) * static_cast<double>(bi.v[j]);
       }
-      bb = team_sum_d<NRHS>(b2, tredd, (nsum_d++) & 1, W, m, bar, nbar, err, redd);
+      if (!team_sum_d<NRHS>(b2, tredd, (nsum_d++) & 1, W, m, bar, nbar, waits, redd))
+        continue;
+      bb = b2;
     }
     const VecN<NRHS> rr0 = rr;
     // per right-hand side stopping threshold on ||r||^2 / ||b||^2: rtol^2,
@@ -548,7 +577,7 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
       tgt[j] = rtol2;
     bool active[NRHS], by_rtol[NRHS];
     int32_t its[NRHS];
-    bool any = false;
+    bool any = false, in_step = true; // in_step: no wait of the team has given up
     int restarts = 0;
 #pragma unroll
     for (int j = 0; j < NRHS; ++j)
@@ -570,7 +599,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
       case 8: pdy = batch_spmv<NRHS, 8>(rowptr, colidx, val, p, y, lo, hi); break;
       default: pdy = batch_spmv<NRHS, 16>(rowptr, colidx, val, p, y, lo, hi); break;
       }
-      pdy = team_total<NRHS>(pdy, words, ++seq, W, m, err, red, total[seq & 1]);
+      ++seq;
+      in_step = team_total<NRHS>(pdy, words, seq, W, m, waits, red, total[seq & 1]);
+      if (!in_step)
+        break;
       float alpha[NRHS];
 #pragma unroll
       for (int j = 0; j < NRHS; ++j)
@@ -592,7 +624,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
         }
         stn<NRHS>(r + o, ri);
       }
-      rn = team_total<NRHS>(rn, words, ++seq, W, m, err, red, total[seq & 1]);
+      ++seq;
+      in_step = team_total<NRHS>(rn, words, seq, W, m, waits, red, total[seq & 1]);
+      if (!in_step)
+        break;
       float beta[NRHS];
       any = false;
 #pragma unroll
@@ -634,9 +669,11 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
         // threshold four times lower (the recursive residual of FP32 CG
         // drifts from the true one by ~1e-7 relative).
         if (W > 1)
-          team_barrier(bar, static_cast<unsigned>(W) * (++nbar), err); // x complete
+          in_step = team_barrier(bar, static_cast<unsigned>(W) * (++nbar), waits); // x complete
         else
           __syncthreads();
+        if (!in_step)
+          break;
         VecD<NRHS> tt;
         switch (g)
         {
@@ -647,7 +684,9 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
         default: tt = batch_resid<NRHS, 16>(rowptr, colidx, val, perm, b, x, r, p, lo, hi); break;
         }
         // (also publishes r and p to the team)
-        tt = team_sum_d<NRHS>(tt, tredd, (nsum_d++) & 1, W, m, bar, nbar, err, redd);
+        in_step = team_sum_d<NRHS>(tt, tredd, (nsum_d++) & 1, W, m, bar, nbar, waits, redd);
+        if (!in_step)
+          break;
         ++restarts;
 #pragma unroll
         for (int j = 0; j < NRHS; ++j)
@@ -680,8 +719,14 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
         stn_agent<NRHS>(p + o, pi);
       }
       if (W > 1)
-        team_publish(bar, static_cast<unsigned>(W) * (++nbar), err); // p complete
+      {
+        in_step = team_publish(bar, static_cast<unsigned>(W) * (++nbar), waits); // p complete
+        if (!in_step)
+          break;
+      }
     }
+    if (!in_step)
+      continue;
     if (perm)
     {
       // this member's rows of x back to the caller's order
@@ -697,10 +742,10 @@ __global__ __launch_bounds__(kMaxBatchBS) void batch_cg_kernel(
   }
 }
 
-// queues = 0, every team's barrier counter and sum words = 0, err = 0 (a kernel, not a
-// memset node, so that graph replays are reliable)
+// queues = 0, every team's barrier counter and sum words = 0, err = 0, iteration counts
+// = -1 (not solved) (a kernel, not a memset node, so that graph replays are reliable)
 __global__ void batch_reset(unsigned* queue, int32_t nq, unsigned* bars, int32_t nsys, int* err,
-                            uint64_t* words, int64_t nwords)
+                            uint64_t* words, int64_t nwords, int32_t* its, int64_t nits)
 {
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nq)
@@ -711,6 +756,8 @@ __global__ void batch_reset(unsigned* queue, int32_t nq, unsigned* bars, int32_t
     bars[k] = 0u;
   for (int64_t k = i; k < nwords; k += gridDim.x * blockDim.x)
     words[k] = 0u;
+  for (int64_t k = i; k < nits; k += gridDim.x * blockDim.x)
+    its[k] = -1;
 }
 
 int pow2_ceil(int v)
@@ -750,6 +797,7 @@ struct spmvx_batch_s
   // systems are the tail of the schedule).
   int32_t rows_per_member = 4096;
   bool members_set = false; // by spmvx_batch_set_config
+  unsigned spin_limit = kSpinLimit;
   int grid = 0;
   // captured graph and the arguments it was captured with
   hipGraphExec_t exec = nullptr;
@@ -994,7 +1042,8 @@ void launch_batch(spmvx_batch_s* B, const float* b, float* x, int32_t max_its, d
   const int32_t* perm = B->reordered ? B->perm.as<int32_t>() : nullptr;
   batch_reset<<<std::max(1, std::min(64, (B->nsys + 255) / 256)), 256, 0, s>>>(
       B->queue.as<unsigned>(), B->nq, B->bars.as<unsigned>(), B->nsys, B->err.as<int>(),
-      B->words.as<uint64_t>(), B->nwords);
+      B->words.as<uint64_t>(), B->nwords, B->its.as<int32_t>(),
+      static_cast<int64_t>(B->nsys) * B->nrhs);
 #define SPMVX_BATCH(NR)                                                                        \
   batch_cg_kernel<NR><<<B->grid, B->block, 0, s>>>(                                           \
       B->rowptr.as<int32_t>(), B->colidx.as<int32_t>(), B->val.as<float>(),                    \
@@ -1003,7 +1052,7 @@ void launch_batch(spmvx_batch_s* B, const float* b, float* x, int32_t max_its, d
       B->tred_off.as<int64_t>(), B->gsel.as<int8_t>(), perm, b, x, xin, r, p, y, max_its,      \
       static_cast<float>(rtol * rtol), rtol * rtol,                                            \
       B->its.as<int32_t>(), B->queue.as<unsigned>(), B->bars.as<unsigned>(),                   \
-      B->tred.as<double>(), B->words.as<uint64_t>(), B->err.as<int>())
+      B->tred.as<double>(), B->words.as<uint64_t>(), B->err.as<int>(), B->spin_limit)
   if (B->nrhs == 4)
     SPMVX_BATCH(4);
   else if (B->nrhs == 2)
@@ -1063,6 +1112,8 @@ int spmvx_batch_create(int32_t nsys, const int32_t* sys_row, const int32_t* rowp
     // solve time by under 1% (the p gathers stay scattered).
     const char* env = std::getenv("SPMVX_BATCH_REORDER");
     B->reordered = env && std::atoi(env) == 1 && nrows > 0;
+    if (const char* spins = std::getenv("SPMVX_BATCH_SPIN_LIMIT"))
+      B->spin_limit = static_cast<unsigned>(std::strtoul(spins, nullptr, 10));
     std::vector<int32_t> nrp, nci, perm;
     std::vector<float> nva;
     if (B->reordered)
