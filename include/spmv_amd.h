@@ -381,9 +381,17 @@ int spmvx_batch_destroy(spmvx_batch B);
 /* Launch configuration: workgroup size (256, 512, 1024), lanes per row
  * (1, 2, 4, 8, 16; 0 = chosen per system from its mean row length) and rows
  * per team member: a system of n rows is solved by a team of
- * ceil(n / rows_per_member) workgroups (capped at 64 and at half the
- * workgroups resident on the device; 0 = one workgroup per system).  Set by
- * the autotuner (spmv_amd/autotune.py). */
+ * ceil(n / rows_per_member) workgroups (capped at 64 and at a sixteenth of the
+ * workgroups resident on the device; 0 = one workgroup per system).  -1, which
+ * a new batch has and spmvx_batch_info then reports, is the default rule:
+ * 4096 rows a member in teams of up to 8, 16384 rows a member beyond, with
+ * the same caps.  Set by the autotuner (spmv_amd/autotune.py).
+ * Batches solved at the same time on several streams: the members of a team
+ * wait for each other, and one solve can have 8 teams of W members waiting for
+ * their last.  k solves are safe while 8 k (W - 1) is below the workgroups
+ * resident on the device (256 of 1024 threads): 4 with teams of 8, 2 with
+ * teams of 16; more may run into the limit of a wait (see
+ * spmvx_batch_solve). */
 int spmvx_batch_set_config(spmvx_batch B, int32_t block, int32_t lanes_per_row,
                            int32_t rows_per_member);
 /*

@@ -590,6 +590,8 @@ class Batch:
             self._h = None
 
     def set_config(self, block, lanes_per_row, rows_per_member=None):
+        """Workgroup size, lanes per row and rows per team member (-1: the default
+        teams; None: as they are, see ``config``)."""
         if rows_per_member is None:
             rows_per_member = self.config()["rows_per_member"]
         _check(lib().spmvx_batch_set_config(self._h, int(block), int(lanes_per_row),

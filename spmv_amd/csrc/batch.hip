@@ -773,6 +773,8 @@ int pow2_ceil(int v)
 
 using namespace spmvx;
 
+constexpr int32_t kDefaultMembers = -1;
+
 struct spmvx_batch_s
 {
   int32_t nsys = 0, nrhs = 0;
@@ -791,12 +793,9 @@ struct spmvx_batch_s
   // launch configuration (autotuned)
   int32_t block = 1024;
   int32_t g_policy = 0;          // 0 = per system from the mean row length, else fixed G
-  // Team size ceil(rows / rows_per_member), 0 = no teams; build_plan has the limits.
-  // 256 systems of 1000 to 50000 rows, 4 right-hand sides, to 1e-6: 16384 rows a member
-  // 126, 8192 81, 4096 66, 2048 66 ms (an exchange costs about 3 us, and the largest
-  // systems are the tail of the schedule).
-  int32_t rows_per_member = 4096;
-  bool members_set = false; // by spmvx_batch_set_config
+  // Team size: ceil(rows / rows_per_member), 0 = no teams, or kDefaultMembers: the
+  // default rule (build_plan has it and the limits).
+  int32_t rows_per_member = kDefaultMembers;
   unsigned spin_limit = kSpinLimit;
   int grid = 0;
   // captured graph and the arguments it was captured with
@@ -942,7 +941,11 @@ int lanes_for(int mean)
   return mean <= 32 ? 4 : std::min(16, pow2_ceil(mean / 8));
 }
 
-constexpr int64_t kSmallTeam = 8, kWideMember = 16384;
+// The default rule for teams: members of kSmallMember rows in teams of up to kSmallTeam,
+// of kWideMember rows beyond.  256 systems of 1000 to 50000 rows, 4 right-hand sides, to
+// 1e-6: 16384 rows a member 126, 8192 81, 4096 66, 2048 66 ms (an exchange costs about 3
+// us, and the largest systems are the tail of the schedule).
+constexpr int64_t kSmallTeam = 8, kSmallMember = 4096, kWideMember = 16384;
 int64_t div_up(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Lanes per row (per system) and the team plan: systems in decreasing size
@@ -970,18 +973,20 @@ void build_plan(spmvx_batch_s* B, int capacity)
       g[s] = static_cast<int8_t>(
           lanes_for(rows > 0 ? static_cast<int>((nz + rows - 1) / rows) : 1));
     }
+    // A launch holds at most one gathering team per queue: 8 (W - 1) workgroups that
+    // wait, with teams of W.  Launches on several streams that together hold all
+    // workgroups that fit the device that way starve each other until the waits run out.
+    // Teams of up to kSmallTeam (56 of the 256 CUs a launch) are safe on the 4 streams
+    // that a process has hardware queues for.  Wider ones are not: systems of more than
+    // 131072 rows, and members chosen by the caller, get teams of up to wmax (16: 120 a
+    // launch, safe on 2 streams).
     int64_t w = 1;
-    if (B->rows_per_member > 0 && B->members_set)
-      // the caller's choice, up to wmax (256 systems of 1000 to 200000 rows, 4096 rows a
-      // member: 453 ms, 530 with the bound below)
-      w = div_up(rows, B->rows_per_member);
+    if (B->rows_per_member == kDefaultMembers)
+      w = std::max(std::min(kSmallTeam, div_up(rows, kSmallMember)), div_up(rows, kWideMember));
     else if (B->rows_per_member > 0)
-      // Members of less than kWideMember rows only in teams of up to kSmallTeam: a
-      // launch holds at most one gathering team per queue, 8 x 7 workgroups, so that
-      // launches on 4 streams (the hardware queues of a process) cannot fill the 256
-      // CUs with teams that all wait for members.
-      w = std::max(std::min(kSmallTeam, div_up(rows, B->rows_per_member)),
-                   div_up(rows, std::max<int64_t>(B->rows_per_member, kWideMember)));
+      // (256 systems of 1000 to 200000 rows, 4096 rows a member: 453 ms, 530 by the
+      // default rule)
+      w = div_up(rows, B->rows_per_member);
     team[s] = static_cast<int32_t>(std::max<int64_t>(1, std::min<int64_t>(w, wmax)));
   }
   // LPT: systems by decreasing work go to the XCD queue with the least work
@@ -1218,14 +1223,13 @@ int spmvx_batch_set_config(spmvx_batch B, int32_t block, int32_t lanes_per_row,
     SPMVX_REQUIRE(lanes_per_row == 0 || lanes_per_row == 1 || lanes_per_row == 2
                       || lanes_per_row == 4 || lanes_per_row == 8 || lanes_per_row == 16,
                   "lanes_per_row must be 0 (per system), 1, 2, 4, 8 or 16");
-    SPMVX_REQUIRE(rows_per_member >= 0, "rows_per_member must be >= 0");
-    if (block != B->block || lanes_per_row != B->g_policy || rows_per_member != B->rows_per_member
-        || !B->members_set)
+    SPMVX_REQUIRE(rows_per_member >= 0 || rows_per_member == kDefaultMembers,
+                  "rows_per_member must be >= 0 (or -1: the default teams)");
+    if (block != B->block || lanes_per_row != B->g_policy || rows_per_member != B->rows_per_member)
     {
       B->block = block;
       B->g_policy = lanes_per_row;
       B->rows_per_member = rows_per_member;
-      B->members_set = true;
       B->plan_dirty = true;
       drop_graph(B);
     }
