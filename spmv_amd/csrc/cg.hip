@@ -124,9 +124,8 @@ template <typename X, typename Acc>
 void ensure_ws(CgWorkspace& w, const Pattern& P, int64_t ncols, int64_t nblocks)
 {
   const int64_t n = P.nrows;
-  const bool small = cg_is_small(P);
-  if (w.mem.ptr && w.n == n && w.ncols == ncols && w.nblocks == nblocks && w.elem == sizeof(X)
-      && (w.p2 != nullptr) == small)
+  const bool small = cg_may_be_small(P);
+  if (w.mem.ptr && w.n == n && w.ncols == ncols && w.nblocks == nblocks && w.elem == sizeof(X))
     return;
   const int vgrid = vec_grid(n > ncols ? n : ncols);
   auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
@@ -244,8 +243,8 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   const V* csr_vals = static_cast<const V*>(A->values.ptr);
   const int g0 = vec_grid(ncols > n ? ncols : n);
   auto* poll = static_cast<CgDevice<Acc>*>(w.poll.ensure(2 * sizeof(CgDevice<double>)));
-  const bool alone = without_exchange(col_map);
-  if (alone && cg_is_tiny(P))
+  const CgForm form = cg_form(P, without_exchange(col_map));
+  if (form.tiny)
     for (bool first = true;; first = false)
     {
       launch_cg_tiny<V, X, Acc>(P, s, csr_vals, b, x, r, p, st, hist_dev, first, kmax, rtol * rtol);
@@ -254,7 +253,7 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
       if (poll->st.stopped)
         return poll->st.k;
     }
-  const bool small = alone && cg_is_small(P);
+  const bool small = form.small;
   if (!w.stream)
   {
     SPMVX_HIP(hipStreamCreateWithFlags(&w.stream, hipStreamNonBlocking));
@@ -285,7 +284,7 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   auto iteration = [&](hipStream_t qq, int j) {
     if (small)
     {
-      launch_small_iteration<V, X, Acc>(P, qq, csr_vals, sm, j + 1);
+      launch_small_iteration<V, X, Acc>(P, form, qq, csr_vals, sm, j + 1);
       return;
     }
     if (col_map)
@@ -305,7 +304,7 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   if (!w.exec || !w.exec_tail || w.g_x != xw || w.g_hist != hist_dev || w.g_map != map_id
       || w.g_halo != halo || w.g_halo_dtype != halo_dt || w.g_variant != A->variant
       || w.g_long_rows != A->long_rows || w.g_mem != w.mem.ptr || w.g_values != vals
-      || w.g_small != (small ? 1 : 0))
+      || w.g_small != (small ? 1 + form.kr : 0))
   {
     for (hipGraphExec_t* e : {&w.exec, &w.exec_tail})
     {
@@ -340,7 +339,7 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
     w.g_long_rows = A->long_rows;
     w.g_mem = w.mem.ptr;
     w.g_values = vals;
-    w.g_small = small ? 1 : 0;
+    w.g_small = small ? 1 + form.kr : 0;
   }
 
   if (small)
@@ -543,9 +542,8 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   double* hist_dev = hist_host ? reinterpret_cast<double*>(base + L.hist) : nullptr;
   const void* vals = sliced ? A->svalues.ptr : A->values.ptr;
   const double* csr_vals = static_cast<const double*>(A->values.ptr);
-  const bool alone = without_exchange(col_map);
-  const bool tiny = alone && cg_is_tiny(P);
-  const bool small = alone && !tiny && cg_is_small(P);
+  const CgForm form = cg_form(P, without_exchange(col_map));
+  const bool tiny = form.tiny, small = form.small;
   const SmallArgs<double, double> sm{
       r,      y,
       {p, reinterpret_cast<double*>(base + kNoAllocBytes + kNoAllocPart)},
@@ -557,7 +555,7 @@ int run_cg_noalloc(spmvx_matrix_s* A, spmvx_l2gmap_s* col_map, const double* b, 
   auto iteration = [&](int j) {
     if (small)
     {
-      launch_small_iteration<double, double, double>(P, s, csr_vals, sm, j + 1);
+      launch_small_iteration<double, double, double>(P, form, s, csr_vals, sm, j + 1);
       return;
     }
     if (col_map)

@@ -524,13 +524,38 @@ __global__ __launch_bounds__(kSmallBS) void cg_residual(int32_t n, X* __restrict
 // 18.4, 30000 (0.29M) 18.6 and 21.4, 100000 (0.96M) 25.3 and 24.9.
 constexpr int64_t kSmallRows = 1024 * 1024;
 constexpr int32_t kSmallWidth = 64;
-inline bool cg_is_small(const Pattern& P)
+// By size alone: what decides about the workspace, which must not change while the
+// masks of a shared pattern are being built.
+inline bool cg_may_be_small(const Pattern& P)
 {
-  if (P.nrows <= 0 || P.nrows > kSmallRows || P.nrows != P.ncols)
-    return false;
+  return P.nrows > 0 && P.nrows <= kSmallRows && P.nrows == P.ncols;
+}
+
+// How a solve iterates: in one workgroup, in two kernels (over the row masks of KR
+// offsets, 0: from colidx), or neither.  Taken once per solve, under the pattern's
+// lock: another thread may be building the masks for another matrix of the pattern.
+struct CgForm
+{
+  bool tiny = false, small = false;
+  int kr = 0;
+};
+inline CgForm cg_form(Pattern& P, bool alone)
+{
+  CgForm f;
+  if (!alone)
+    return f;
+  f.tiny = cg_is_tiny(P);
+  if (f.tiny || !cg_may_be_small(P))
+    return f;
+  std::lock_guard<std::recursive_mutex> lock(P.lazy_mu);
   if (P.masked && P.all_masked)
-    return P.nnz <= (kWaveClasses[P.wave].kr <= 9 ? 6000000 : 2000000);
-  return P.longest <= kSmallWidth && P.nnz <= 600000;
+  {
+    f.kr = kWaveClasses[P.wave].kr;
+    f.small = P.nnz <= (f.kr <= 9 ? 6000000 : 2000000);
+  }
+  else
+    f.small = P.longest <= kSmallWidth && P.nnz <= 600000;
+  return f;
 }
 
 inline int small_blocks(int64_t n) { return static_cast<int>((n + kSmallBS - 1) / kSmallBS); }
@@ -551,10 +576,10 @@ struct SmallArgs
   Acc* hist;
 };
 
-// Iteration j (its parity matters) on stream s.
+// Iteration j (its parity matters) on stream s, in the form f.
 template <typename V, typename X, typename Acc>
-void launch_small_iteration(Pattern& P, hipStream_t s, const V* val, const SmallArgs<X, Acc>& a,
-                            int j)
+void launch_small_iteration(const Pattern& P, const CgForm& f, hipStream_t s, const V* val,
+                            const SmallArgs<X, Acc>& a, int j)
 {
   const int32_t n = static_cast<int32_t>(P.nrows);
   const int par = j & 1;
@@ -565,7 +590,7 @@ void launch_small_iteration(Pattern& P, hipStream_t s, const V* val, const Small
         small_partials(n), a.part_s, a.st, a.slot + (par ^ 1), a.slot + par, a.hist);
   };
   using std::integral_constant;
-  switch (P.masked && P.all_masked ? kWaveClasses[P.wave_class()].kr : 0)
+  switch (f.kr)
   {
   case 3: go(integral_constant<int, 3>{}); break;
   case 5: go(integral_constant<int, 5>{}); break;

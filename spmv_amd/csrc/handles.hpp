@@ -298,7 +298,7 @@ struct CgWorkspace
   hipGraph_t graph_tail = nullptr; // kTailChunk iterations (near convergence)
   hipGraphExec_t exec_tail = nullptr;
   const void* g_x = nullptr;   // arguments the graphs were captured with
-  int32_t g_small = -1;
+  int32_t g_small = -1; // two-kernel iterations: 1 + their mask width, else 0
   const void* g_hist = nullptr;
   uint64_t g_map = 0; // id of the column map (0: none)
   const void* g_halo = nullptr;

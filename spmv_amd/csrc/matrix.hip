@@ -502,6 +502,7 @@ CsrView csr_view(Pattern& P, int var, size_t vbytes)
 
 CsrView csr_view_built(Pattern& P, int var, size_t vbytes)
 {
+  std::lock_guard<std::recursive_mutex> lock(P.lazy_mu);
   const RowBlocks* rb = built_variant_blocks(P, var);
   return make_view(P, rb && variant_short(var) && !rb->short_built ? nullptr : rb, var, vbytes);
 }
