@@ -243,6 +243,13 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
   const V* csr_vals = static_cast<const V*>(A->values.ptr);
   const int g0 = vec_grid(ncols > n ? ncols : n);
   auto* poll = static_cast<CgDevice<Acc>*>(w.poll.ensure(2 * sizeof(CgDevice<double>)));
+  if (col_map)
+  {
+    l2gmap_prepare_device(col_map);
+    // checked for every form of the iteration, not first inside the captured iterations
+    SPMVX_REQUIRE(col_map->halo_dtype < 0 || col_map->halo_dtype == vec_dtype,
+                  "halo dtype differs from the vector dtype");
+  }
   const CgForm form = cg_form(P, without_exchange(col_map));
   if (form.tiny)
     for (bool first = true;; first = false)
@@ -262,13 +269,6 @@ int run_cg(spmvx_matrix_s* A, CgWorkspace& w, spmvx_l2gmap_s* col_map, int32_t v
     SPMVX_HIP(hipEventCreateWithFlags(&w.ev_poll[1], hipEventDisableTiming));
   }
   hipStream_t q = w.stream;
-  if (col_map)
-  {
-    l2gmap_prepare_device(col_map);
-    // checked here, not first inside the captured iterations
-    SPMVX_REQUIRE(col_map->halo_dtype < 0 || col_map->halo_dtype == vec_dtype,
-                  "halo dtype differs from the vector dtype");
-  }
   const bool sliced = A->variant == kSlicedVariant;
   const SlicedView sv = sliced ? sliced_view(A) : SlicedView{};
   const void* vals = sliced ? A->svalues.ptr : A->values.ptr;
