@@ -602,7 +602,8 @@ int pattern_default_variant(Pattern& P, int32_t dtype)
     return base;
   if (is_complex(dtype))
   {
-    (void)complex_wave(P, dtype, base);
+    if (!complex_wave(P, dtype, base))
+      (void)variant_blocks(P, base);
     return base;
   }
   // the short-index kernel for the dtype when the matrix fits it (the
