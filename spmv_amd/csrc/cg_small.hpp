@@ -212,7 +212,8 @@ __global__ __launch_bounds__(kTinyBS) void cg_tiny(
       const int32_t i = t + j * kTinyBS;
       xv[j] = xv[j] + al * lp[i < n ? i : n];
       rv[j] = rv[j] - al * yv[j];
-      rn += static_cast<Acc>(rv[j]) * static_cast<Acc>(rv[j]);
+      // (past the last row an infinite alpha has made a NaN of 0 - alpha 0)
+      rn += i < n ? static_cast<Acc>(rv[j]) * static_cast<Acc>(rv[j]) : Acc(0);
     }
     rn = group_total<NW>(rn, red[1]);
     const X be = static_cast<X>(rn / rr);
