@@ -177,15 +177,20 @@ int spmvx_matrix_arrays(spmvx_matrix A, const int32_t** rowptr_dev,
  * streaming loads, index width; 0 <= variant < spmvx_num_kernels(), -1 =
  * the matrix's default).  All variants give identical results; used by
  * tuning.  No reference counterpart (the inspector of Matrix.cpp:43 picks its
- * own kernel).  Variants 8-11 read 16-bit column indices: for every row block
- * whose columns fall into at most four windows of 16384 columns (stencils,
+ * own kernel).  Variants 8-11 read 16-bit column indices: where the columns of
+ * every row block fall into at most four windows of 16384 columns (stencils,
  * banded and locally numbered matrices) the analysis stores each column as a
- * window number and an offset (2 instead of 4 bytes per entry); other blocks
- * keep the 32-bit indices.  A matrix's default is the 16-bit counterpart of
- * its dtype's default kernel when that covers at least half of the entries.
- * Variants 8, 10 and 11 (those defaults) give every 64 rows to one wavefront
- * where the rows are short and alike, and keep, for matrices whose rows use a
- * short common list of column offsets, a mask per row in the indices' place.
+ * window number and an offset (2 instead of 4 bytes per entry); SPMVX_ERR_ARG
+ * for a matrix that does not fit.  The default of a matrix that does is one of
+ * them.  Variants 8, 10 and 11 give every 64 rows to one wavefront where the
+ * rows are short and alike, and keep, for matrices whose rows use a short
+ * common list of column offsets, a mask per row in the indices' place.  For
+ * complex values variant 1 (SPMVX_C64) and variant 2 (SPMVX_C32), the defaults,
+ * do the same where every row has such a mask, also when they are chosen here;
+ * 0, 3 and 4 never do.
+ * The variant is that of the products.  CG of a system without ghosts of up to
+ * about a million rows iterates with kernels of its own, whatever the variant
+ * (see spmvx_cg); the sums of a row stay in stored order.
  * The last variant, SPMVX_SLICED_VARIANT, is the sliced row-pattern layout:
  * for matrices whose rows repeat a few column-offset patterns (stencils), a
  * copy of the values is kept in 64-row slices with a 16-bit pattern id per
@@ -251,6 +256,12 @@ int spmvx_spmv_t(spmvx_matrix A, const void* x_dev, void* y_dev, spmvx_stream st
  * direction vector every iteration (cg.cpp:55) through the transport above.
  *   b_dev[nrows], x_dev[ncols] (ghost entries returned as 0), *its = k.
  *   hist_host (may be NULL): max_its+1 doubles, hist[j] = ||r_j||^2.
+ * Systems without ghosts or indices to pack are solved in one workgroup (up to
+ * 4096 rows, up to 56 entries a row on 512 rows and 7 on 4096) or with two
+ * kernels per iteration (up to 2^20 rows: 6 million entries with row masks over
+ * at most 9 column offsets, 2 million with more, 600 thousand and 64 a row
+ * without masks); A's kernel variant and its long-row mode have no part in
+ * those.
  * Errors: "spmv::cg - Error: b.rows() != A.rows()" style argument checks.
  */
 int spmvx_cg(spmvx_matrix A, spmvx_l2gmap col_map, const double* b_dev, double* x_dev,
@@ -264,12 +275,14 @@ int spmvx_cg(spmvx_matrix A, spmvx_l2gmap col_map, const double* b_dev, double* 
  * checks and results as spmvx_cg (the same kernels in the same order: x, *its
  * and the history are bit-identical), but every buffer of the solve (r, A p,
  * the direction vector, partial sums, the device-side scalars and the
- * history) lives in a fixed device array of SPMVX_CG_NOALLOC_SCRATCH_BYTES
- * that the library holds on every GPU it runs on until the process ends, and
- * the kernels are launched directly on `stream` (no captured graph, no
- * internal stream or event).  The call needs about 8 * (2 * nrows + ncols)
- * bytes plus 8 * (max_its + 1) with a history; a solve that needs more is
- * rejected with SPMVX_ERR_ARG before any kernel runs.  Preconditions (else
+ * history) lives in a fixed device array that the library holds on every GPU
+ * it runs on until the process ends, and the kernels are launched directly on
+ * `stream` (no captured graph, no internal stream or event).  The call needs
+ * about 8 * (2 * nrows + ncols) bytes plus 8 * (max_its + 1) with a history; a
+ * solve that needs more than SPMVX_CG_NOALLOC_SCRATCH_BYTES is rejected with
+ * SPMVX_ERR_ARG before any kernel runs.  The array itself takes
+ * SPMVX_CG_NOALLOC_RESIDENT_BYTES on every GPU: the partial sums of some
+ * kernels and a second direction have room behind that limit.  Preconditions (else
  * SPMVX_ERR_ARG, nothing launched): the row blocks of A's kernel variant and,
  * for the sliced variant, its layout exist (spmvx_matrix_create and
  * spmvx_matrix_set_kernel build them), and a col_map with ghosts or pack
@@ -279,6 +292,7 @@ int spmvx_cg(spmvx_matrix A, spmvx_l2gmap col_map, const double* b_dev, double* 
  * must be serialised by the caller.  Synchronises `stream`.
  */
 #define SPMVX_CG_NOALLOC_SCRATCH_BYTES (32u << 20)
+#define SPMVX_CG_NOALLOC_RESIDENT_BYTES ((40u << 20) + (128u << 10))
 int spmvx_cg_noalloc(spmvx_matrix A, spmvx_l2gmap col_map, const double* b_dev, double* x_dev,
                      int32_t max_its, double rtol, int32_t* its, double* hist_host,
                      spmvx_stream stream);

@@ -435,7 +435,9 @@ static_assert(kNoAllocParts >= size_t(kWaveMaxGrid), "one partial sum per wavefr
 constexpr size_t kNoAllocPart = sizeof(double) * kNoAllocParts;
 // the second direction of the two-kernel iteration
 constexpr size_t kNoAllocSmall = sizeof(double) * kSmallRows;
-static __device__ __align__(256) unsigned char scratch[kNoAllocBytes + kNoAllocPart + kNoAllocSmall];
+static_assert(kNoAllocBytes + kNoAllocPart + kNoAllocSmall == SPMVX_CG_NOALLOC_RESIDENT_BYTES,
+              "what the header says the scratch takes");
+static __device__ __align__(256) unsigned char scratch[SPMVX_CG_NOALLOC_RESIDENT_BYTES];
 
 constexpr int kMaxDevices = 64;
 std::mutex scratch_mu;

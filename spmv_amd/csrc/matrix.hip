@@ -567,6 +567,8 @@ bool small_blocks_suit(const Pattern& P, int32_t dtype)
 // in flight.  us with 8192 and 2048 entries a block: transposed assembly maps, 6.5
 // million entries 28.1 and 25.0, 8.4 million 36.9 and 31.6, 18 million 65.9 and 62.9, 72
 // million 298 and 291; random rows, 4.8 million 40.9 and 36.4, 38 million 600 and 578.
+// (Repeated products, which find what fits in the last-level cache; one product after 2 GiB
+// of other writes, 8.4 million entries, with its launch: 49.2 and 42.7.)
 // A matrix's own product keeps 8192 above the limit: CG sums its blocks' partials.
 int plain_variant(const Pattern& P, int32_t dtype)
 {
